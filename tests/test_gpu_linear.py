@@ -203,3 +203,13 @@ def test_fused_gate_up_silu_routing_and_fallback(gpu):
     assert not ops.uses_silu_kernel(0, 256, 256) and not ops.uses_decode_kernel(0, 512, 256)
     assert ops.linear_silu_mul(x0[:0], w0).shape == (0, 256)
     assert ops.linear(x0[:0], w0).shape == (0, 512)
+
+
+@pytest.mark.parametrize("m", [1, 128, 130, 256])
+@pytest.mark.parametrize("n,k,config,splits", [(512, 64, 6, 1), (768, 320, 0, 1), (512, 1280, 7, 4),
+                                               (1536, 192, 6, 1), (768, 832, 7, 1)])
+def test_k_phases(gpu, m, n, k, config, splits):
+    """N / 2 a multiple of the tile: every tile starts at its own K step and wraps, with fewer
+    steps than phases, step counts that are no power of two, and one or several M tiles."""
+    x, w = operands(m, n, k, torch.bfloat16, gpu, m + n + k)
+    check_product(ops.decode_linear(x, w, config=config, splits=splits), x, w)
