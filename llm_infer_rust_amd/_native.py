@@ -101,6 +101,10 @@ SIGNATURES: dict[str, tuple] = {
                                           c_void_p]),
     "mi355x_sample": (c_char_p, [c_void_p, c_i64, c_i64, c_i64, c_int, c_void_p, c_void_p,
                                  c_void_p, c_u64, c_u64, c_void_p, c_void_p]),
+    "mi355x_sample_split": (c_char_p, [c_void_p, c_i64, c_i64, c_i64, c_int, c_void_p, c_void_p,
+                                       c_void_p, c_u64, c_u64, c_void_p, c_bool, c_void_p,
+                                       c_i64, c_void_p]),
+    "mi355x_sample_workspace_bytes": (c_i64, [c_i64, c_i64, c_bool]),
 }
 
 _lock = threading.Lock()

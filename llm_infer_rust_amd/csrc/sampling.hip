@@ -35,6 +35,8 @@
 //     SC'11) keyed by the seed, with counter (element/4, row, offset), so the
 //     draw needs no prefix scan and no renormalising sum.
 // Without either cutoff only the race pass runs; greedy rows run one argmax pass.
+#include <cfloat>
+
 #include "common.h"
 
 namespace mi355x {
@@ -215,10 +217,106 @@ __device__ void block_scan(Shared& sh, uint32_t& c, unsigned long long& m, uint3
   __syncthreads();
 }
 
+__device__ __forceinline__ float probability(float s, float m, float inv_z) {
+  return exp2f((s - m) * kLog2e) * inv_z;
+}
+__device__ __forceinline__ unsigned long long fixed_mass(float p) {
+  return static_cast<unsigned long long>(p * kFixedScale + 0.5f);
+}
+// Mass that the top-p cutoff has to reach: at least one unit, so the top bin is selectable.
+__device__ __forceinline__ unsigned long long mass_target(float top_p) {
+  const unsigned long long t = static_cast<unsigned long long>(top_p * kFixedScale);
+  return t ? t : 1ull;
+}
+// Below the k-th largest scaled logit by far more than the rounding of p: every token under
+// this edge has a p strictly below the k-th largest p.
+__device__ __forceinline__ float candidate_edge(float s_k, float m) {
+  return s_k - (fabsf(s_k - m) + 1.f) * 0x1p-12f;
+}
+
+// Both cutoffs and the draw among n gathered candidates (cand_p is scratch; the lists are in
+// LDS and complete: every token of the row whose p can reach the k-th largest is listed).
+// False, and nothing written, when fewer than k candidates exist or the k-th p has no
+// fixed-point mass under a top-p cutoff. All kThreads threads call it.
+__device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& a, int64_t row,
+                                                  const uint32_t* cand_i, const float* cand_s,
+                                                  float* cand_p, uint32_t n, float m, float inv_z,
+                                                  int64_t top_k, float top_p) {
+  const bool use_p = top_p < 1.f;
+  const unsigned long long p_target = mass_target(top_p);
+  for (uint32_t t = threadIdx.x; t < n; t += kThreads)
+    cand_p[t] = probability(cand_s[t], m, inv_z);
+  if (threadIdx.x == 0) sh.k_found = 0;
+  __syncthreads();
+  // The k-th largest p: the candidate value v with #(p > v) < k <= #(p >= v).
+  for (uint32_t t = threadIdx.x; t < n; t += kThreads) {
+    const float v = cand_p[t];
+    uint32_t gt = 0, ge = 0;
+    for (uint32_t u = 0; u < n; ++u) {
+      gt += cand_p[u] > v;
+      ge += cand_p[u] >= v;
+    }
+    if (gt < static_cast<uint32_t>(top_k) && ge >= static_cast<uint32_t>(top_k)) {
+      sh.red_f[0] = v;  // every thread that gets here writes the same value
+      sh.k_found = 1;
+    }
+  }
+  __syncthreads();
+  const float p_k = sh.red_f[0];
+  if (!sh.k_found || (use_p && fixed_mass(p_k) == 0)) return false;
+  float cut = p_k;
+  if (use_p) {
+    // Mass at or above p_k; when it reaches top_p, the top-p cutoff is the largest
+    // candidate value whose mass at or above reaches it.
+    unsigned long long mk = 0;
+    for (uint32_t t = threadIdx.x; t < n; t += kThreads)
+      if (cand_p[t] >= p_k) mk += fixed_mass(cand_p[t]);
+    uint32_t zc = 0;
+    uint32_t tc;
+    unsigned long long tm;
+    block_scan(sh, zc, mk, tc, tm);
+    if (tm >= p_target) {
+      float best_v = p_k;
+      for (uint32_t t = threadIdx.x; t < n; t += kThreads) {
+        const float v = cand_p[t];
+        if (v < p_k) continue;
+        unsigned long long mv = 0;
+        for (uint32_t u = 0; u < n; ++u)
+          if (cand_p[u] >= v) mv += fixed_mass(cand_p[u]);
+        if (mv >= p_target) best_v = fmaxf(best_v, v);
+      }
+      float bv = best_v;
+      int64_t bi = 0;
+      block_argmax(sh, bv, bi);
+      cut = bv;
+    }
+  }
+  // The race over the surviving candidates (order-independent: larger key, then lower index).
+  float best = -INFINITY;
+  int64_t best_i = a.vocab;
+  for (uint32_t t = threadIdx.x; t < n; t += kThreads) {
+    const float pt = cand_p[t];
+    if (!(pt > 0.f && pt >= cut)) continue;
+    const int64_t i = cand_i[t];
+    const uint4 rnd =
+        philox4x32_10(make_uint4(static_cast<uint32_t>(i >> 2), static_cast<uint32_t>(row),
+                                 a.offset_lo, a.offset_hi),
+                      a.seed_lo, a.seed_hi);
+    const uint32_t words[4] = {rnd.x, rnd.y, rnd.z, rnd.w};
+    const float key = cand_s[t] + gumbel(words[i & 3]);
+    if (key > best || (key == best && i < best_i)) {
+      best = key;
+      best_i = i;
+    }
+  }
+  block_argmax(sh, best, best_i);
+  if (threadIdx.x == 0) a.out[row] = best_i < a.vocab ? best_i : -1;
+  return true;
+}
+
+// One whole row by one workgroup.
 template <int DT>
-__global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec) {
-  __shared__ Shared sh;
-  const int64_t row = blockIdx.x;
+__device__ __forceinline__ void sample_row(Shared& sh, const SampleArgs& a, int64_t row, bool vec) {
   const int64_t vocab = a.vocab;
 
   float temperature = a.temperature[row];
@@ -338,13 +436,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
     }
   }
   const float inv_z = 1.f / z;
-  auto prob = [&](float s) { return exp2f((s - m) * kLog2e) * inv_z; };
-  auto fixed = [](float p) { return static_cast<unsigned long long>(p * kFixedScale + 0.5f); };
+  auto prob = [&](float s) { return probability(s, m, inv_z); };
   const bool use_p = top_p < 1.f;
-  const unsigned long long p_target = [&] {
-    const unsigned long long t = static_cast<unsigned long long>(top_p * kFixedScale);
-    return t ? t : 1ull;  // at least one unit, so the top bin is always selectable
-  }();
+  const unsigned long long p_target = mass_target(top_p);
 
   // Candidate path (top-k rows): the order-key histogram of pass 1 gives the bin b1 that
   // holds the k-th largest scaled logit. Every token with s >= s_lo (the bin's lower edge
@@ -380,8 +474,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
     __syncthreads();
     bool ok = sh.k_found && sh.k_rem <= kCandidates;
     if (ok) {
-      const float s_lower = key_value(sh.k_prefix << 20);
-      const float s_lo = s_lower - (fabsf(s_lower - m) + 1.f) * 0x1p-12f;
+      const float s_lo = candidate_edge(key_value(sh.k_prefix << 20), m);
       uint32_t* cand_i = reinterpret_cast<uint32_t*>(sh.mass);
       float* cand_s = reinterpret_cast<float*>(cand_i + kCandidates);
       float* cand_p = cand_s + kCandidates;
@@ -400,77 +493,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
       const uint32_t n = sh.p_lowest;
       ok = n <= kCandidates;
       if (ok) {
-        for (uint32_t t = threadIdx.x; t < n; t += kThreads) cand_p[t] = prob(cand_s[t]);
-        __syncthreads();
-        // The k-th largest p: the candidate value v with #(p > v) < k <= #(p >= v).
-        if (threadIdx.x == 0) sh.k_found = 0;
-        __syncthreads();
-        for (uint32_t t = threadIdx.x; t < n; t += kThreads) {
-          const float v = cand_p[t];
-          uint32_t gt = 0, ge = 0;
-          for (uint32_t u = 0; u < n; ++u) {
-            gt += cand_p[u] > v;
-            ge += cand_p[u] >= v;
-          }
-          if (gt < static_cast<uint32_t>(top_k) && ge >= static_cast<uint32_t>(top_k)) {
-            sh.red_f[0] = v;  // every thread that gets here writes the same value
-            sh.k_found = 1;
-          }
-        }
-        __syncthreads();
-        const float p_k = sh.red_f[0];
-        ok = sh.k_found && !(use_p && fixed(p_k) == 0);
-        float cut = p_k;
-        if (ok && use_p) {
-          // Mass at or above p_k; when it reaches top_p, the top-p cutoff is the largest
-          // candidate value whose mass at or above reaches it.
-          unsigned long long mk = 0;
-          for (uint32_t t = threadIdx.x; t < n; t += kThreads)
-            if (cand_p[t] >= p_k) mk += fixed(cand_p[t]);
-          uint32_t zc = 0;
-          uint32_t tc;
-          unsigned long long tm;
-          block_scan(sh, zc, mk, tc, tm);
-          if (tm >= p_target) {
-            float best_v = p_k;
-            for (uint32_t t = threadIdx.x; t < n; t += kThreads) {
-              const float v = cand_p[t];
-              if (v < p_k) continue;
-              unsigned long long mv = 0;
-              for (uint32_t u = 0; u < n; ++u)
-                if (cand_p[u] >= v) mv += fixed(cand_p[u]);
-              if (mv >= p_target) best_v = fmaxf(best_v, v);
-            }
-            float bv = best_v;
-            int64_t bi = 0;
-            block_argmax(sh, bv, bi);
-            cut = bv;
-          }
-        }
-        if (ok) {
-          // The race over the surviving candidates (order-independent: larger key, then
-          // lower index).
-          float best = -INFINITY;
-          int64_t best_i = vocab;
-          for (uint32_t t = threadIdx.x; t < n; t += kThreads) {
-            const float pt = cand_p[t];
-            if (!(pt > 0.f && pt >= cut)) continue;
-            const int64_t i = cand_i[t];
-            const uint4 rnd =
-                philox4x32_10(make_uint4(static_cast<uint32_t>(i >> 2), static_cast<uint32_t>(row),
-                                         a.offset_lo, a.offset_hi),
-                              k0, k1);
-            const uint32_t words[4] = {rnd.x, rnd.y, rnd.z, rnd.w};
-            const float key = cand_s[t] + gumbel(words[i & 3]);
-            if (key > best || (key == best && i < best_i)) {
-              best = key;
-              best_i = i;
-            }
-          }
-          block_argmax(sh, best, best_i);
-          if (threadIdx.x == 0) a.out[row] = best_i < vocab ? best_i : -1;
+        if (finish_candidates(sh, a, row, cand_i, cand_s, cand_p, n, m, inv_z, top_k, top_p))
           return;
-        }
       }
     }
     __syncthreads();  // the candidate lists alias the mass histogram of the radix path
@@ -511,7 +535,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
       const uint32_t hi = above >= 32 ? 0u : key >> above;
       if (use_k && hi == kp) atomicAdd(&sh.cnt[bin], 1u);
       if (use_p && hi == pp) {
-        const unsigned long long fx = static_cast<unsigned long long>(p * kFixedScale + 0.5f);
+        const unsigned long long fx = fixed_mass(p);
         if (fx) atomicAdd(&sh.mass[bin], fx);
       }
     });
@@ -577,6 +601,959 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
   if (threadIdx.x == 0) a.out[row] = best_i < vocab ? best_i : -1;
 }
 
+template <int DT>
+__global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec) {
+  __shared__ Shared sh;
+  sample_row<DT>(sh, a, blockIdx.x, vec);
+}
+
+// ---------------------------------------------------------------------------
+// A row over several workgroups. One workgroup per row leaves the chip idle for a handful of
+// rows and walks a row two to five times; here every workgroup holds one segment of a row in
+// registers, so the logits are read once for greedy, unfiltered and top-k rows. Bound by
+// VALU work where the rows are many (an exponential per logit; 256 rows of 151,936 bf16 logits,
+// top-k 50 and top-p 0.9: 26 + 16 us a call against 66 with one workgroup per row), by latency
+// and launches where they are few (5 mixed rows 197 -> 50 us, 5 top-k rows 72 -> 23):
+//   sample_segments  per segment: the argmax, or the race's best token, or the segment's max
+//                    and sum of exp(s - max); top-k rows also list the tokens at or above a
+//                    bound on the segment's k-th largest (the k-th largest of the 256 threads'
+//                    maxima);
+//   mass_level       rows cut by top-p alone: mass histograms over the order key of s, a few
+//                    bits per launch, each launch picking the bin that holds the cutoff in the
+//                    previous launch's histogram (p grows with s, so the cutoff on s is the
+//                    cutoff on p);
+//   race_segments    those rows' race over the survivors, per segment;
+//   sample_finish    one workgroup per row joins the segments. Rows whose lists overflow (heavy
+//                    ties) or whose parameters fit none of the above take sample_row.
+// Cutoffs and draws are sample_row's: masses are the same fixed-point sums, the race is the
+// same, and the sum of exp differs by its fp32 rounding only.
+// ---------------------------------------------------------------------------
+constexpr int kSegThreads = 256;
+constexpr int kSegWarps = kSegThreads / kWave;
+constexpr int kChunk = kSegThreads * 8;   // elements a workgroup takes per step
+constexpr int kMaxChunks = 4;             // steps held in registers (8: half the waves fit)
+constexpr int kMaxSegments = 256;         // per row
+constexpr uint32_t kSegList = 512;        // listed tokens per segment
+constexpr int64_t kSplitTopK = 128;       // largest k of the segment lists
+constexpr uint32_t kRowList = 8192;       // listed tokens per row
+constexpr int kSegPeaks = kSegThreads / 16;
+constexpr int kLevelBins = 1024;          // bins of the levels after the first
+
+enum class Rule { kGreedy, kRace, kTopK, kTopP, kWhole };
+
+struct RowRule {
+  Rule rule;
+  float temperature, top_p;
+  int64_t top_k;
+};
+
+__device__ __forceinline__ RowRule row_rule(const SampleArgs& a, int64_t row, bool top_p_rows) {
+  RowRule r;
+  r.temperature = a.temperature[row];
+  r.top_p = a.top_p[row];
+  if (!(r.top_p >= 0.f && r.top_p <= 1.f)) r.top_p = 1.f;
+  r.top_k = a.top_k[row];
+  if (r.top_k <= 0 || r.top_k > a.vocab) r.top_k = a.vocab;
+  if (r.temperature <= 0.f || r.top_p == 0.f)
+    r.rule = Rule::kGreedy;
+  else if (r.top_k == a.vocab)
+    r.rule = r.top_p < 1.f ? (top_p_rows ? Rule::kTopP : Rule::kWhole) : Rule::kRace;
+  else
+    r.rule = r.top_k <= kSplitTopK ? Rule::kTopK : Rule::kWhole;
+  return r;
+}
+
+struct Segment {
+  float m, z;         // max of s and sum of exp(s - m)
+  float bound;        // top-k rows: every token with s >= bound is listed
+  uint32_t count;     // listed tokens (more than kSegList: the list is incomplete)
+  float best;         // argmax value or race key
+  uint32_t best_i;    // its index; vocab when the segment has none
+  uint32_t bad;       // a NaN or +inf among s
+  uint32_t pad;
+};
+
+struct LevelState {
+  uint32_t prefix, pad;
+  unsigned long long rem;
+};
+
+struct SplitArgs {
+  Segment* seg;              // [rows][segments]
+  float* peak;               // [rows][segments][kSegPeaks]: maxima of 16 threads each
+  uint2* list;               // [rows][segments][kSegList]: (index, bits of s)
+  LevelState* state;         // [rows][4]
+  unsigned long long* hist;  // [rows][kBins0 + 2 kLevelBins], top_p_rows only
+  int32_t segments;
+  bool vec, top_p_rows;
+};
+constexpr int64_t kHistWords = kBins0 + 2 * kLevelBins;
+
+// Bits of the order key told apart by each level: all the bits a logit of the type can differ
+// in (fp16 values have 10 mantissa bits of fp32's 23 and more exponents in their denormals).
+template <int DT>
+__device__ __forceinline__ constexpr int level_bits(int level) {
+  if (level == 0) return 12;
+  return DT == 0 ? 4 : DT == 1 ? 7 : 10;
+}
+template <int DT>
+constexpr int kLevels = DT == 2 ? 3 : 2;
+
+// max(a, b, c) in one instruction; a NaN among them is passed over. (fmaxf spends a second
+// instruction on each operand, for signalling NaNs.)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// The chunk's 8 logits of this thread. Elements past the row are -inf, before and after scaling.
+// VEC: 16-byte aligned rows of a multiple of 8 logits, so 8 are all inside or all past the row.
+template <int DT, bool VEC>
+struct Chunk {
+  using W = typename Logit<DT>::Word;
+  static constexpr int kWords = DT == 2 ? 2 : 1;
+  static constexpr uint32_t kNone = DT == 0 ? 0xff80ff80u : DT == 1 ? 0xfc00fc00u : 0xff800000u;
+  uint4 raw[kWords];
+  __device__ __forceinline__ void load(const SampleArgs& a, int64_t row, uint32_t e) {
+    const W* base = static_cast<const W*>(a.logits) + row * a.stride;
+    const uint32_t vocab = static_cast<uint32_t>(a.vocab);
+#pragma unroll
+    for (int j = 0; j < kWords; ++j) raw[j] = make_uint4(kNone, kNone, kNone, kNone);
+    if constexpr (VEC) {
+      if (e < vocab) {
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) raw[j] = ld128(base + e + j * (8 / kWords));
+      }
+    } else {
+      W v[8];
+      __builtin_memcpy(v, raw, sizeof(v));
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (e + j < vocab) v[j] = base[e + j];
+      __builtin_memcpy(raw, v, sizeof(raw));
+    }
+  }
+  __device__ __forceinline__ void values(float (&f)[8]) const {
+    if constexpr (DT == 2) {
+      __builtin_memcpy(f, raw, sizeof(f));
+    } else {
+      unpack8<DT>(raw[0], f);
+    }
+  }
+  // Replaces the logits by the scaled logits s; returns their maximum (NaN aside). Rounding
+  // keeps order, so the largest product rounds to the largest s.
+  __device__ __forceinline__ float scale(float inv_t, uint32_t e, uint32_t vocab) {
+    float f[8];
+    values(f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      f[j] = f[j] * inv_t;
+      if constexpr (DT == 2) f[j] = Logit<2>::round(f[j]);
+      if constexpr (!VEC)
+        if (e + j >= vocab) f[j] = -INFINITY;  // -inf times 0 (an infinite temperature) is NaN
+    }
+    float top = max3(max3(max3(f[0], f[1], f[2]), f[3], f[4]), max3(f[5], f[6], f[7]), -INFINITY);
+    top = Logit<DT>::round(top);
+    if constexpr (DT == 2)
+      __builtin_memcpy(raw, f, sizeof(f));
+    else
+      raw[0] = pack8<DT>(f);
+    if constexpr (VEC)
+      if (e >= vocab) {
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) raw[j] = make_uint4(kNone, kNone, kNone, kNone);
+        top = -INFINITY;
+      }
+    return top;
+  }
+  // Forgets what the compiler knows of the values, so that a later pass unpacks them again
+  // rather than keeping 8 floats a chunk alive.
+  __device__ __forceinline__ void repack() {
+#pragma unroll
+    for (int j = 0; j < kWords; ++j)
+      asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
+  }
+};
+
+struct alignas(16) SegShared {
+  float peak[kSegThreads];
+  float red_f[kSegWarps];
+  uint32_t red_i[kSegWarps];
+  float bound;
+  uint32_t count;
+};
+
+// The k-th largest of a wave's values, 4 per lane, by the 16 top bits of their order keys (so at
+// least k of them reach the result); -inf when fewer than k are finite. One ballot per value
+// and bit: no LDS and no barriers.
+__device__ __forceinline__ float kth_largest(const float (&v)[4], uint32_t k) {
+  uint32_t key[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) key[t] = v[t] == -INFINITY ? 0u : order_key(v[t]);
+  uint32_t found = 0;
+#pragma unroll
+  for (int b = 31; b >= 16; --b) {
+    const uint32_t next = found | (1u << b);
+    uint32_t c = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) c += __popcll(__ballot(key[t] >= next));
+    found = c >= k ? next : found;
+  }
+  return found ? key_value(found) : -INFINITY;
+}
+
+__device__ __forceinline__ float wave_max(float x) {
+  x = row16_max(x);
+  x = fmaxf(x, __shfl_xor(x, 16));
+  return fmaxf(x, __shfl_xor(x, 32));
+}
+
+// Workgroup best (value, index) of a segment: larger value, then lower index; NaN above all.
+__device__ __forceinline__ void segment_best(SegShared& sh, float& v, uint32_t& i) {
+  const int lane = threadIdx.x % kWave, warp = threadIdx.x / kWave;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const float ov = __shfl_xor(v, off);
+    const uint32_t oi = __shfl_xor(i, off);
+    if (better(ov, oi, v, i)) {
+      v = ov;
+      i = oi;
+    }
+  }
+  if (lane == 0) {
+    sh.red_f[warp] = v;
+    sh.red_i[warp] = i;
+  }
+  __syncthreads();
+  v = sh.red_f[0];
+  i = sh.red_i[0];
+  for (int w = 1; w < kSegWarps; ++w)
+    if (better(sh.red_f[w], sh.red_i[w], v, i)) {
+      v = sh.red_f[w];
+      i = sh.red_i[w];
+    }
+}
+
+// Race keys of 8 neighbouring tokens starting at e; `keep` tells which take part.
+template <typename Keep>
+__device__ __forceinline__ void race8(const SampleArgs& a, int64_t row, uint32_t e,
+                                      const float (&s)[8], Keep&& keep, float& best,
+                                      uint32_t& best_i) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) any = any || keep(s[4 * h + j]);
+    if (!any) continue;
+    const uint4 rnd =
+        philox4x32_10(make_uint4((e >> 2) + h, static_cast<uint32_t>(row),
+                                 a.offset_lo, a.offset_hi),
+                      a.seed_lo, a.seed_hi);
+    const uint32_t words[4] = {rnd.x, rnd.y, rnd.z, rnd.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (!keep(s[4 * h + j])) continue;
+      const float key = s[4 * h + j] + gumbel(words[j]);
+      const uint32_t i = e + 4 * h + j;
+      if (key > best || (key == best && i < best_i)) {
+        best = key;
+        best_i = i;
+      }
+    }
+  }
+}
+
+// Max and sum of exp over a row's segments. Every wave that calls it gets the same bits.
+// False for an invalid distribution (NaN, +inf, or nothing finite).
+__device__ __forceinline__ bool join_segments(const Segment* seg, int n, float& m, float& z) {
+  const int lane = threadIdx.x % kWave;
+  m = -INFINITY;
+  bool bad = false;
+  for (int j = lane; j < n; j += kWave) {
+    m = fmaxf(m, seg[j].m);
+    bad = bad || seg[j].bad;
+  }
+  m = wave_max(m);
+  z = 0.f;
+  for (int j = lane; j < n; j += kWave)
+    if (seg[j].m != -INFINITY) z += seg[j].z * exp2f((seg[j].m - m) * kLog2e);
+  z = wave_sum(z);
+  return !__any(bad) && m != -INFINITY && z > 0.f;
+}
+
+template <int DT, int NCH, bool VEC>
+__global__ __launch_bounds__(kSegThreads) void sample_segments(SampleArgs a, SplitArgs p) {
+  __shared__ SegShared sh;
+  const int64_t row = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid % kWave, warp = tid / kWave;
+  const RowRule r = row_rule(a, row, p.top_p_rows);
+  if (r.rule == Rule::kWhole) return;  // sample_finish takes the row whole
+  // Indexes fit 32 bits: a split row has at most kMaxSegments * kMaxChunks * kChunk elements.
+  const uint32_t vocab = static_cast<uint32_t>(a.vocab);
+  const uint32_t e0 = blockIdx.x * uint32_t(NCH * kChunk) + tid * 8;
+  Segment* out = p.seg + row * p.segments + blockIdx.x;
+
+  // Unfiltered rows stream their chunks (the race's random words would crowd out chunks held in
+  // registers).
+  if (r.rule == Rule::kRace) {
+    const float inv_t = 1.f / r.temperature;
+    float best = -INFINITY;
+    uint32_t best_i = vocab;
+    bool bad = false;
+    Chunk<DT, VEC> next;
+    next.load(a, row, e0);
+#pragma unroll 1
+    for (int c = 0; c < NCH; ++c) {
+      Chunk<DT, VEC> x = next;
+      const uint32_t e = e0 + c * kChunk;
+      if (c + 1 < NCH) next.load(a, row, e + kChunk);
+      float s[8];
+      x.scale(inv_t, e, vocab);
+      x.values(s);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) bad = bad || !(s[j] < INFINITY);
+      race8(a, row, e, s, [](float v) { return v > -INFINITY; }, best, best_i);
+    }
+    const int any_bad = __syncthreads_or(bad);
+    segment_best(sh, best, best_i);
+    if (tid == 0) {
+      out->best = best;
+      out->best_i = best_i;
+      out->bad = any_bad;
+    }
+    return;
+  }
+
+  if (r.rule == Rule::kTopP) {
+    // The row's histograms for the next launches, cleared by its segments together.
+    unsigned long long* h = p.hist + row * kHistWords;
+    for (int64_t i = int64_t(blockIdx.x) * kSegThreads + tid; i < kHistWords;
+         i += int64_t(p.segments) * kSegThreads)
+      h[i] = 0;
+  }
+  Chunk<DT, VEC> x[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) x[c].load(a, row, e0 + c * kChunk);
+
+  if (r.rule == Rule::kGreedy) {
+    // A thread looks for its first maximum chunk by chunk, and element by element only in
+    // chunks that raise it or hold a NaN (their sum is one).
+    float best = -INFINITY;
+    uint32_t best_i = vocab;  // any real index beats the sentinel
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      float f[8];
+      x[c].values(f);
+      const uint32_t e = e0 + c * kChunk;
+      const float top = max3(max3(max3(f[0], f[1], f[2]), f[3], f[4]), max3(f[5], f[6], f[7]), best);
+      const float sum = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+      if (best_i != vocab && !(top > best) && sum == sum) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (e + j < vocab && better(f[j], e + j, best, best_i)) {
+          best = f[j];
+          best_i = e + j;
+        }
+    }
+    segment_best(sh, best, best_i);
+    if (tid == 0) {
+      out->best = best;
+      out->best_i = best_i;
+    }
+    return;
+  }
+
+  const float inv_t = 1.f / r.temperature;
+  float cm[NCH], tm = -INFINITY;  // maxima per chunk and thread, then of the workgroup
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    cm[c] = x[c].scale(inv_t, e0 + c * kChunk, vocab);
+    tm = max3(tm, cm[c], -INFINITY);
+    x[c].repack();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const bool listed = r.rule == Rule::kTopK;
+  const float rm = row16_max(tm);
+  float wm = fmaxf(rm, __shfl_xor(rm, 16));
+  wm = fmaxf(wm, __shfl_xor(wm, 32));
+  if (lane == 0) sh.red_f[warp] = wm;
+  if (listed) {
+    sh.peak[tid] = tm;
+    if (lane % 16 == 0)
+      p.peak[(row * p.segments + blockIdx.x) * kSegPeaks + tid / 16] = rm;
+    if (tid == 0) sh.count = 0;
+  }
+  __syncthreads();
+  float m = sh.red_f[0];
+  for (int w = 1; w < kSegWarps; ++w) m = fmaxf(m, sh.red_f[w]);
+  if (m == -INFINITY || m == INFINITY) {  // nothing finite, or a +inf: only a NaN is to be found
+    bool bad = m == INFINITY;
+    for (int c = 0; c < NCH; ++c) {
+      float s[8];
+      x[c].values(s);
+      for (int j = 0; j < 8; ++j) bad = bad || s[j] != s[j];
+    }
+    const int any_bad = __syncthreads_or(bad);
+    if (tid == 0) *out = Segment{m, 0.f, 0.f, 0u, 0.f, vocab, static_cast<uint32_t>(any_bad), 0u};
+    return;
+  }
+  if (listed && warp == 0) {
+    // At least k tokens of the segment reach the k-th largest of its threads' maxima.
+    const float4 v4 = *reinterpret_cast<const float4*>(sh.peak + 4 * lane);
+    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+    const float t = kth_largest(v, static_cast<uint32_t>(r.top_k));
+    if (lane == 0) sh.bound = t == -INFINITY ? -FLT_MAX : t - (fabsf(t - m) + 1.f) * 0x1p-11f;
+  }
+
+  // fp32 sums with the hardware exponential: a term it flushes to zero lies below 2^-126
+  // beside the maximum's own 1.
+  float z = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    float s[8];
+    x[c].values(s);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) z += __builtin_amdgcn_exp2f((s[j] - m) * kLog2e);
+    x[c].repack();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float bound = 0.f;
+  if (listed) {
+    __syncthreads();
+    bound = sh.bound;
+    uint2* list = p.list + (row * p.segments + blockIdx.x) * int64_t(kSegList);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if (cm[c] >= bound) {
+        float s[8];
+        x[c].values(s);
+        uint32_t hits = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) hits |= s[j] >= bound ? 1u << j : 0u;
+        while (hits) {
+          const uint32_t j = __builtin_ctz(hits);
+          hits &= hits - 1;
+          float v = s[0];
+#pragma unroll
+          for (uint32_t t = 1; t < 8; ++t) v = j == t ? s[t] : v;
+          const uint32_t slot = atomicAdd(&sh.count, 1u);
+          if (slot < kSegList) list[slot] = make_uint2(e0 + c * kChunk + j, __float_as_uint(v));
+        }
+      }
+    }
+  }
+  z = wave_sum(z);
+  __syncthreads();  // red_f's readers are done; the list is complete
+  if (lane == 0) sh.red_f[warp] = z;
+  __syncthreads();
+  if (tid == 0) {
+    z = (sh.red_f[0] + sh.red_f[1]) + (sh.red_f[2] + sh.red_f[3]);
+    *out = Segment{m, z, bound, sh.count, 0.f, vocab, z != z ? 1u : 0u, 0u};  // a NaN among s
+  }
+}
+
+// Scan of the previous level's histogram by one workgroup of kSegThreads: the bin where the
+// mass from the top reaches st.rem joins the prefix; when rounding keeps every prefix below it,
+// the lowest bin that holds mass.
+template <int NBINS>
+__device__ __forceinline__ LevelState next_state(const unsigned long long* hist, LevelState st,
+                                                 int bits, unsigned long long* sh_m,
+                                                 uint32_t* sh_bin, unsigned long long* sh_rem) {
+  constexpr int kOwn = NBINS / kSegThreads;
+  const int tid = threadIdx.x, lane = tid % kWave, warp = tid / kWave;
+  unsigned long long own[kOwn], sum = 0;
+  int lowest = NBINS;
+#pragma unroll
+  for (int j = kOwn - 1; j >= 0; --j) {
+    own[j] = hist[tid * kOwn + j];
+    sum += own[j];
+    if (own[j]) lowest = tid * kOwn + j;
+  }
+  unsigned long long incl = sum;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const unsigned long long o = __shfl_down(incl, off);
+    if (lane + off < kWave) incl += o;
+  }
+  if (tid == 0) *sh_bin = NBINS;
+  if (lane == 0) sh_m[warp] = incl;
+  __syncthreads();
+  unsigned long long above = incl - sum, total = 0;
+  for (int w = 0; w < kSegWarps; ++w) {
+    if (w > warp) above += sh_m[w];
+    total += sh_m[w];
+  }
+  if (total < st.rem) {
+    if (lowest < NBINS) atomicMin(sh_bin, static_cast<uint32_t>(lowest));
+    __syncthreads();
+    const uint32_t b = *sh_bin < NBINS ? *sh_bin : 0u;
+    return LevelState{(st.prefix << bits) | b, 0u, hist[b]};
+  }
+#pragma unroll
+  for (int j = kOwn - 1; j >= 0; --j) {
+    if (own[j] && above < st.rem && above + own[j] >= st.rem) {
+      *sh_bin = static_cast<uint32_t>(tid * kOwn + j);
+      *sh_rem = st.rem - above;
+    }
+    above += own[j];
+  }
+  __syncthreads();
+  return LevelState{(st.prefix << bits) | *sh_bin, 0u, *sh_rem};
+}
+
+struct LevelShared {
+  unsigned long long mass[kBins0];
+  unsigned long long sum[kSegWarps];
+  unsigned long long rem;
+  uint32_t bin;
+};
+
+// The state after `level` histograms (level >= 1), kept by the row's first segment.
+template <int DT>
+__device__ __forceinline__ LevelState level_state(const SplitArgs& p, int64_t row, int level,
+                                                  LevelShared& sh) {
+  const unsigned long long* h = p.hist + row * kHistWords;
+  LevelState* st = p.state + row * 4;
+  const LevelState prev = st[level - 1];
+  const LevelState now =
+      level == 1 ? next_state<kBins0>(h, prev, level_bits<DT>(0), sh.sum, &sh.bin, &sh.rem)
+                 : next_state<kLevelBins>(h + kBins0 + (level - 2) * kLevelBins, prev,
+                                          level_bits<DT>(level - 1), sh.sum, &sh.bin, &sh.rem);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st[level] = now;
+  return now;
+}
+
+template <int DT, int LEVEL, bool VEC>
+__global__ __launch_bounds__(kSegThreads) void mass_level(SampleArgs a, SplitArgs p, int chunks) {
+  __shared__ LevelShared sh;
+  const int64_t row = blockIdx.y;
+  const RowRule r = row_rule(a, row, p.top_p_rows);
+  if (r.rule != Rule::kTopP) return;
+  float m, z;
+  if (!join_segments(p.seg + row * p.segments, p.segments, m, z)) return;
+  constexpr int kNBins = LEVEL == 0 ? kBins0 : kLevelBins;
+  uint32_t prefix = 0;
+  if constexpr (LEVEL > 0)
+    prefix = level_state<DT>(p, row, LEVEL, sh).prefix;
+  else if (blockIdx.x == 0 && threadIdx.x == 0)
+    p.state[row * 4] = LevelState{0u, 0u, mass_target(r.top_p)};
+  for (int b = threadIdx.x; b < kNBins; b += kSegThreads) sh.mass[b] = 0;
+  __syncthreads();
+  constexpr int kAbove = LEVEL == 0 ? 32 : LEVEL == 1 ? 20 : 20 - level_bits<DT>(1);
+  constexpr int kBits = level_bits<DT>(LEVEL);
+  const float inv_z = 1.f / z, inv_t = 1.f / r.temperature;
+  const uint32_t vocab = static_cast<uint32_t>(a.vocab);
+  const uint32_t e0 = blockIdx.x * uint32_t(chunks * kChunk) + threadIdx.x * 8;
+  for (int c = 0; c < chunks; ++c) {
+    const uint32_t e = e0 + c * kChunk;
+    if (e >= vocab) break;
+    Chunk<DT, VEC> x;
+    x.load(a, row, e);
+    x.scale(inv_t, e, vocab);
+    float s[8];
+    x.values(s);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t key = order_key(s[j]);
+      if (LEVEL > 0 && key >> (kAbove & 31) != prefix) continue;
+      const unsigned long long fx = fixed_mass(probability(s[j], m, inv_z));  // 0 for -inf
+      if (fx) atomicAdd(&sh.mass[key >> (kAbove - kBits) & ((1u << kBits) - 1u)], fx);
+    }
+  }
+  __syncthreads();
+  unsigned long long* h =
+      p.hist + row * kHistWords + (LEVEL == 0 ? 0 : kBins0 + (LEVEL - 1) * kLevelBins);
+  for (int b = threadIdx.x; b < (1 << kBits); b += kSegThreads)
+    if (sh.mass[b]) atomicAdd(&h[b], sh.mass[b]);
+}
+
+template <int DT, bool VEC>
+__global__ __launch_bounds__(kSegThreads) void race_segments(SampleArgs a, SplitArgs p,
+                                                             int chunks) {
+  __shared__ LevelShared sh;
+  __shared__ SegShared sg;
+  const int64_t row = blockIdx.y;
+  const RowRule r = row_rule(a, row, p.top_p_rows);
+  if (r.rule != Rule::kTopP) return;
+  float m, z;
+  if (!join_segments(p.seg + row * p.segments, p.segments, m, z)) return;
+  constexpr int kShift = 20 - (kLevels<DT> - 1) * level_bits<DT>(1);
+  const uint32_t prefix = level_state<DT>(p, row, kLevels<DT>, sh).prefix;
+  // The cutoff's s: the prefix's bits, the others as they are in every value of the type.
+  uint32_t key = prefix << kShift;
+  if (!(key & 0x80000000u)) key |= (1u << kShift) - 1u;
+  const float s_cut = key_value(key);
+  const float inv_z = 1.f / z, inv_t = 1.f / r.temperature;
+  const float cut = probability(s_cut, m, inv_z);
+  const float edge = candidate_edge(s_cut, m);  // no token below it has a p that reaches cut
+  const uint32_t vocab = static_cast<uint32_t>(a.vocab);
+  const uint32_t e0 = blockIdx.x * uint32_t(chunks * kChunk) + threadIdx.x * 8;
+  float best = -INFINITY;
+  uint32_t best_i = vocab;
+  for (int c = 0; c < chunks; ++c) {
+    const uint32_t e = e0 + c * kChunk;
+    if (e >= vocab) break;
+    Chunk<DT, VEC> x;
+    x.load(a, row, e);
+    x.scale(inv_t, e, vocab);
+    float s[8];
+    x.values(s);
+    race8(a, row, e, s,
+          [&](float v) {
+            if (!(v >= edge)) return false;
+            const float q = probability(v, m, inv_z);
+            return q > 0.f && q >= cut;
+          },
+          best, best_i);
+  }
+  segment_best(sg, best, best_i);
+  if (threadIdx.x == 0) {
+    Segment* out = p.seg + row * p.segments + blockIdx.x;
+    out->best = best;
+    out->best_i = best_i;
+  }
+}
+
+// finish_candidates for at most 64 R candidates by one wave, each pair compared through lane
+// broadcasts: with 60 candidates 4 us against the workgroup-wide version's 16 (its LDS round
+// trips). False as well when tokens that could share the k-th p may not have been listed, the
+// lists being complete down to listed_to only.
+template <int R>
+__device__ bool finish_wave(const SampleArgs& a, int64_t row, const uint32_t* cand_i,
+                            const float* cand_s, uint32_t n, float m, float inv_z, int64_t top_k,
+                            float top_p, float listed_to) {
+  const int lane = threadIdx.x % kWave;
+  const bool use_p = top_p < 1.f;
+  const uint32_t k = static_cast<uint32_t>(top_k);
+  float s[R], p[R];
+  uint32_t gt[R], ge[R];
+  unsigned long long fx[R], mass[R];  // mass at or above the own p
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const uint32_t c = lane + kWave * t;
+    s[t] = c < n ? cand_s[c] : -INFINITY;
+    p[t] = c < n ? probability(s[t], m, inv_z) : -1.f;
+    fx[t] = c < n ? fixed_mass(p[t]) : 0ull;
+    gt[t] = ge[t] = 0;
+    mass[t] = 0;
+  }
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const int some = min(kWave, static_cast<int>(n) - kWave * t);
+    for (int u = 0; u < some; ++u) {
+      const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p[t]), u));
+      const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx[t]), u);
+      const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx[t] >> 32), u);
+      const unsigned long long f = (static_cast<unsigned long long>(hi) << 32) | lo;
+#pragma unroll
+      for (int w = 0; w < R; ++w) {
+        gt[w] += v > p[w];
+        const bool above = v >= p[w];
+        ge[w] += above;
+        mass[w] += above ? f : 0ull;
+      }
+    }
+  }
+  // The k-th largest p and the mass at or above it.
+  float p_k = -1.f;
+  bool reached = false;
+#pragma unroll
+  for (int t = 0; t < R; ++t)
+    if (p[t] >= 0.f && gt[t] < k && ge[t] >= k) {
+      p_k = p[t];
+      reached = mass[t] >= mass_target(top_p);
+    }
+  reached = __any(reached);
+  p_k = wave_max(p_k);
+  if (p_k < 0.f || (use_p && fixed_mass(p_k) == 0)) return false;
+  float s_k = INFINITY;  // the lowest s that has it
+#pragma unroll
+  for (int t = 0; t < R; ++t)
+    if (p[t] == p_k) s_k = fminf(s_k, s[t]);
+  s_k = -wave_max(-s_k);
+  if (listed_to > candidate_edge(s_k, m)) return false;
+  float cut = p_k;
+  if (use_p && reached) {
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      if (p[t] > cut && mass[t] >= mass_target(top_p)) cut = p[t];
+    cut = wave_max(cut);
+  }
+  float best = -INFINITY;
+  uint32_t best_i = static_cast<uint32_t>(a.vocab);
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    if (!(p[t] > 0.f && p[t] >= cut)) continue;
+    const uint32_t i = cand_i[lane + kWave * t];
+    const uint4 rnd = philox4x32_10(
+        make_uint4(i >> 2, static_cast<uint32_t>(row), a.offset_lo, a.offset_hi), a.seed_lo,
+        a.seed_hi);
+    const uint32_t w01 = i & 1 ? rnd.y : rnd.x, w23 = i & 1 ? rnd.w : rnd.z;
+    const float key = s[t] + gumbel(i & 2 ? w23 : w01);
+    if (key > best || (key == best && i < best_i)) {
+      best = key;
+      best_i = i;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const float ov = __shfl_xor(best, off);
+    const uint32_t oi = __shfl_xor(best_i, off);
+    if (ov > best || (ov == best && oi < best_i)) {
+      best = ov;
+      best_i = oi;
+    }
+  }
+  if (lane == 0) a.out[row] = best_i < a.vocab ? static_cast<int64_t>(best_i) : -1;
+  return true;
+}
+
+struct alignas(16) FinishShared {
+  Segment seg[kMaxSegments];
+  uint32_t offset[kMaxSegments];
+  uint32_t count;
+  float edge;
+  int ok;
+  Shared row;
+};
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArgs p) {
+  __shared__ FinishShared sh;
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid % kWave, warp = tid / kWave;
+  const int n = p.segments;
+  if (tid < 2 * n)  // two 16-byte halves per segment
+    reinterpret_cast<uint4*>(sh.seg)[tid] =
+        reinterpret_cast<const uint4*>(p.seg + row * p.segments)[tid];
+  const RowRule r = row_rule(a, row, p.top_p_rows);
+  if (r.rule == Rule::kWhole) {
+    sample_row<DT>(sh.row, a, row, p.vec);
+    return;
+  }
+  __syncthreads();
+  const Segment* seg = sh.seg;
+  if (r.rule != Rule::kTopK) {
+    bool bad = false;
+    if (r.rule == Rule::kTopP) {
+      float m, z;
+      bad = !join_segments(seg, n, m, z);
+    }
+    float best = -INFINITY;
+    int64_t best_i = a.vocab;
+    if (!bad && tid < n) {
+      best = seg[tid].best;
+      best_i = seg[tid].best_i;
+      if (r.rule == Rule::kRace) bad = seg[tid].bad != 0;
+    }
+    const int any_bad = __syncthreads_or(bad);
+    block_argmax(sh.row, best, best_i);
+    if (tid == 0) {
+      if (r.rule == Rule::kGreedy)
+        a.out[row] = best_i < a.vocab ? best_i : 0;
+      else
+        a.out[row] = any_bad || best_i >= a.vocab ? -1 : best_i;
+    }
+    return;
+  }
+
+  float m, z;
+  if (!join_segments(seg, n, m, z)) {
+    if (tid == 0) a.out[row] = -1;
+    return;
+  }
+  // Top-k: every wave finds the offsets of the segments' lists in the row's (the same values
+  // into the same words) and loads its tokens; meanwhile one wave takes a lower bound of the
+  // k-th largest s from the segments' peaks, folded into 256 groups. The tokens that reach the
+  // bound, little more than k, are kept for finish_candidates' work.
+  const uint32_t k = static_cast<uint32_t>(r.top_k);
+  uint32_t total = 0;
+  bool full = false;
+  for (int j0 = 0; j0 < n; j0 += kWave) {
+    const int j = j0 + lane;
+    const uint32_t c = j < n ? seg[j].count : 0;
+    full = full || c > kSegList;
+    uint32_t incl = c;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t o = __shfl_up(incl, off);
+      if (lane >= off) incl += o;
+    }
+    if (j < n) sh.offset[j] = total + incl - c;
+    total += __shfl(incl, kWave - 1);
+  }
+  bool ok = !__any(full) && total >= k && total <= kRowList;  // the same in every wave
+  if (ok) {
+    constexpr int kOwn = kRowList / kThreads;
+    const uint2* lists = p.list + row * n * int64_t(kSegList);
+    uint2 own[kOwn];
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) {
+      const uint32_t i = tid + t * kThreads;
+      if (i >= total) break;
+      int lo = 0, hi = n;  // the last segment whose list starts at or before i
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (sh.offset[mid] <= i)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      own[t] = lists[lo * int64_t(kSegList) + (i - sh.offset[lo])];
+    }
+    if (warp == 0) {
+      const float* peak = p.peak + row * n * kSegPeaks;
+      float v[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      for (int i = 4 * lane; i < kSegPeaks * n; i += 4 * kWave) {
+        const float4 q = *reinterpret_cast<const float4*>(peak + i);
+        v[0] = fmaxf(v[0], q.x);
+        v[1] = fmaxf(v[1], q.y);
+        v[2] = fmaxf(v[2], q.z);
+        v[3] = fmaxf(v[3], q.w);
+      }
+      const float t = kth_largest(v, k);
+      if (lane == 0) {
+        sh.edge = t == -INFINITY ? -FLT_MAX : candidate_edge(t, m);
+        sh.count = 0;
+      }
+    }
+    __syncthreads();
+    const float edge = sh.edge;
+    uint32_t* cand_i = reinterpret_cast<uint32_t*>(sh.row.mass);
+    float* cand_s = reinterpret_cast<float*>(cand_i + kCandidates);
+    float* cand_p = cand_s + kCandidates;
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) {
+      if (tid + t * kThreads >= total) break;
+      const float s = __uint_as_float(own[t].y);
+      if (!(s >= edge)) continue;
+      const uint32_t slot = atomicAdd(&sh.count, 1u);
+      if (slot < kCandidates) {
+        cand_i[slot] = own[t].x;
+        cand_s[slot] = s;
+      }
+    }
+    float listed_to = -FLT_MAX;
+    for (int j = lane; j < n; j += kWave)
+      if (seg[j].m != -INFINITY) listed_to = fmaxf(listed_to, seg[j].bound);
+    listed_to = wave_max(listed_to);
+    __syncthreads();
+    const uint32_t kept = sh.count;
+    if (kept <= 4 * kWave) {
+      // What is left fits one wave's registers.
+      if (warp == 0) {
+        const float inv_z = 1.f / z;
+        const bool done =
+            kept <= kWave
+                ? finish_wave<1>(a, row, cand_i, cand_s, kept, m, inv_z, r.top_k, r.top_p, listed_to)
+            : kept <= 2 * kWave
+                ? finish_wave<2>(a, row, cand_i, cand_s, kept, m, inv_z, r.top_k, r.top_p, listed_to)
+                : finish_wave<4>(a, row, cand_i, cand_s, kept, m, inv_z, r.top_k, r.top_p,
+                                 listed_to);
+        if (lane == 0) sh.ok = done;
+      }
+      __syncthreads();
+      ok = sh.ok != 0;
+    } else {
+      // The whole workgroup, where the bound itself shows the lists complete.
+      ok = kept <= kCandidates && listed_to <= edge &&
+           finish_candidates(sh.row, a, row, cand_i, cand_s, cand_p, kept, m, 1.f / z, r.top_k,
+                             r.top_p);
+    }
+  }
+  if (ok) return;
+  __syncthreads();
+  sample_row<DT>(sh.row, a, row, p.vec);
+}
+
+// How a call is split: chunks of kChunk logits per workgroup, workgroups per row. More chunks
+// (fewer lists to join) while they still give 1,024 workgroups, four per CU, and kMinSegments
+// segments, whose peaks bound the k-th largest for every k of the lists. Rows of up to 8 chunks
+// are quicker in one launch (2,300 logits, top-k 50: 18 us against 27), and above 1,024 rows one
+// workgroup per row fills the chip by itself.
+constexpr int kMinSegments = 9;
+static_assert(kMinSegments * kSegPeaks >= kSplitTopK, "a bound for every k");
+struct SplitPlan {
+  int chunks, segments;  // segments 0: one workgroup per row (sample_kernel)
+};
+
+SplitPlan split_plan(int64_t rows, int64_t vocab) {
+  const int64_t total = (vocab + kChunk - 1) / kChunk;
+  int chunks = 1;
+  if (rows > 1024 || total < kMinSegments) return {0, 0};
+  auto count = [&](int c) { return (total + c - 1) / c; };
+  while (chunks < kMaxChunks &&
+         ((rows * count(2 * chunks) >= 1024 && count(2 * chunks) >= kMinSegments) ||
+          count(chunks) > kMaxSegments))
+    chunks *= 2;
+  const int64_t segments = count(chunks);
+  if (segments > kMaxSegments) return {0, 0};
+  return {chunks, static_cast<int>(segments)};
+}
+
+template <int DT, bool VEC>
+void launch_segments(const SampleArgs& a, const SplitArgs& p, int chunks, hipStream_t s) {
+  const dim3 grid(static_cast<uint32_t>(p.segments), static_cast<uint32_t>(a.rows));
+  const dim3 block(kSegThreads);
+  switch (chunks) {
+    case 1: sample_segments<DT, 1, VEC><<<grid, block, 0, s>>>(a, p); break;
+    case 2: sample_segments<DT, 2, VEC><<<grid, block, 0, s>>>(a, p); break;
+    default: sample_segments<DT, kMaxChunks, VEC><<<grid, block, 0, s>>>(a, p); break;
+  }
+  if (p.top_p_rows) {
+    mass_level<DT, 0, VEC><<<grid, block, 0, s>>>(a, p, chunks);
+    mass_level<DT, 1, VEC><<<grid, block, 0, s>>>(a, p, chunks);
+    if constexpr (kLevels<DT> > 2) mass_level<DT, 2, VEC><<<grid, block, 0, s>>>(a, p, chunks);
+    race_segments<DT, VEC><<<grid, block, 0, s>>>(a, p, chunks);
+  }
+}
+
+template <int DT>
+void launch_split(const SampleArgs& a, const SplitArgs& p, int chunks, hipStream_t s) {
+  if (p.vec && a.vocab % 8 == 0)
+    launch_segments<DT, true>(a, p, chunks, s);
+  else
+    launch_segments<DT, false>(a, p, chunks, s);
+  sample_finish<DT><<<dim3(static_cast<uint32_t>(a.rows)), dim3(kThreads), 0, s>>>(a, p);
+}
+
+int64_t round256(int64_t n) { return (n + 255) / 256 * 256; }
+
+// Checks shared by the two entries; fills the arguments. `done`: nothing to launch.
+const char* sample_args(const void* logits, int64_t rows, int64_t vocab, int64_t row_stride,
+                        int dtype, const float* temperature, const int32_t* top_k,
+                        const float* top_p, uint64_t seed, uint64_t offset, int64_t* out,
+                        SampleArgs* a, bool* vec, bool* done) {
+  *done = false;
+  if (rows < 0 || vocab <= 0 || row_stride < vocab) return set_error("mi355x_sample: bad shape");
+  if (vocab >= (int64_t(1) << 32) || rows >= (int64_t(1) << 31))
+    return set_error("mi355x_sample: shape too large");
+  if (dtype < 0 || dtype > 2)
+    return set_error("mi355x_sample: dtype must be 0 (bf16), 1 (fp16) or 2 (fp32)");
+  if (rows == 0) {
+    *done = true;
+    return nullptr;
+  }
+  if (!logits || !temperature || !top_k || !top_p || !out)
+    return set_error("mi355x_sample: null pointer");
+  a->logits = logits;
+  a->rows = rows;
+  a->vocab = vocab;
+  a->stride = row_stride;
+  a->temperature = temperature;
+  a->top_k = top_k;
+  a->top_p = top_p;
+  a->seed_lo = static_cast<uint32_t>(seed);
+  a->seed_hi = static_cast<uint32_t>(seed >> 32);
+  a->offset_lo = static_cast<uint32_t>(offset);
+  a->offset_hi = static_cast<uint32_t>(offset >> 32);
+  a->out = out;
+  const int per_vec = dtype == 2 ? 4 : 8;
+  *vec = aligned(logits, 16) && row_stride % per_vec == 0;
+  return nullptr;
+}
+
 }  // namespace
 }  // namespace mi355x
 
@@ -586,29 +1563,12 @@ extern "C" const char* mi355x_sample(const void* logits, int64_t rows, int64_t v
                                      int64_t row_stride, int dtype, const float* temperature,
                                      const int32_t* top_k, const float* top_p, uint64_t seed,
                                      uint64_t offset, int64_t* out, void* stream) {
-  if (rows < 0 || vocab <= 0 || row_stride < vocab) return set_error("mi355x_sample: bad shape");
-  if (vocab >= (int64_t(1) << 32) || rows >= (int64_t(1) << 31))
-    return set_error("mi355x_sample: shape too large");
-  if (dtype < 0 || dtype > 2)
-    return set_error("mi355x_sample: dtype must be 0 (bf16), 1 (fp16) or 2 (fp32)");
-  if (rows == 0) return nullptr;
-  if (!logits || !temperature || !top_k || !top_p || !out)
-    return set_error("mi355x_sample: null pointer");
   SampleArgs a{};
-  a.logits = logits;
-  a.rows = rows;
-  a.vocab = vocab;
-  a.stride = row_stride;
-  a.temperature = temperature;
-  a.top_k = top_k;
-  a.top_p = top_p;
-  a.seed_lo = static_cast<uint32_t>(seed);
-  a.seed_hi = static_cast<uint32_t>(seed >> 32);
-  a.offset_lo = static_cast<uint32_t>(offset);
-  a.offset_hi = static_cast<uint32_t>(offset >> 32);
-  a.out = out;
-  const int per_vec = dtype == 2 ? 4 : 8;
-  const bool vec = aligned(logits, 16) && row_stride % per_vec == 0;
+  bool vec = false, done = false;
+  if (const char* e = sample_args(logits, rows, vocab, row_stride, dtype, temperature, top_k,
+                                  top_p, seed, offset, out, &a, &vec, &done))
+    return e;
+  if (done) return nullptr;
   auto s = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<uint32_t>(rows));
   if (dtype == 0)
@@ -618,4 +1578,55 @@ extern "C" const char* mi355x_sample(const void* logits, int64_t rows, int64_t v
   else
     sample_kernel<2><<<grid, dim3(kThreads), 0, s>>>(a, vec);
   return launch_status("mi355x_sample");
+}
+
+extern "C" int64_t mi355x_sample_workspace_bytes(int64_t rows, int64_t vocab, bool top_p_rows) {
+  if (rows <= 0 || vocab <= 0 || vocab >= (int64_t(1) << 32)) return 0;
+  const int64_t n = rows * split_plan(rows, vocab).segments;
+  if (n == 0) return 0;
+  return round256(n * int64_t(sizeof(Segment))) + n * kSegPeaks * 4 + n * kSegList * int64_t(sizeof(uint2)) +
+         round256(rows * 4 * int64_t(sizeof(LevelState))) +
+         (top_p_rows ? rows * kHistWords * 8 : 0);
+}
+
+extern "C" const char* mi355x_sample_split(const void* logits, int64_t rows, int64_t vocab,
+                                           int64_t row_stride, int dtype,
+                                           const float* temperature, const int32_t* top_k,
+                                           const float* top_p, uint64_t seed, uint64_t offset,
+                                           int64_t* out, bool top_p_rows, void* workspace,
+                                           int64_t workspace_bytes, void* stream) {
+  SampleArgs a{};
+  bool vec = false, done = false;
+  if (const char* e = sample_args(logits, rows, vocab, row_stride, dtype, temperature, top_k,
+                                  top_p, seed, offset, out, &a, &vec, &done))
+    return e;
+  if (done) return nullptr;
+  const SplitPlan plan = split_plan(rows, vocab);
+  if (plan.segments == 0) return set_error("mi355x_sample_split: shape not split");
+  if (!workspace || !aligned(workspace, 16) ||
+      workspace_bytes < mi355x_sample_workspace_bytes(rows, vocab, top_p_rows))
+    return set_error("mi355x_sample_split: workspace too small");
+  SplitArgs p{};
+  const int64_t n = rows * plan.segments;
+  auto* base = static_cast<uint8_t*>(workspace);
+  p.seg = reinterpret_cast<Segment*>(base);
+  base += round256(n * int64_t(sizeof(Segment)));
+  p.peak = reinterpret_cast<float*>(base);
+  base += n * kSegPeaks * 4;
+  p.list = reinterpret_cast<uint2*>(base);
+  base += n * kSegList * int64_t(sizeof(uint2));
+  p.state = reinterpret_cast<LevelState*>(base);
+  base += round256(rows * 4 * int64_t(sizeof(LevelState)));
+  p.hist = reinterpret_cast<unsigned long long*>(base);
+  p.segments = plan.segments;
+  p.vec = vec;
+  p.top_p_rows = top_p_rows;
+  auto s = static_cast<hipStream_t>(stream);
+  if (dtype == 0)
+    launch_split<0>(a, p, plan.chunks, s);
+  else if (dtype == 1)
+    launch_split<1>(a, p, plan.chunks, s);
+  else
+    launch_split<2>(a, p, plan.chunks, s);
+  return launch_status("mi355x_sample_split");
 }

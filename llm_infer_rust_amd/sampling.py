@@ -43,6 +43,14 @@ class SamplingParams:
         return replace(self, max_tokens=max(self.max_tokens, 1), top_p=top_p)
 
 
+# The split sampler cuts rows with a top_k up to this among their listed largest logits. A
+# larger one below the vocabulary takes one workgroup per row from the start (k 200, 64 rows of
+# 151,936: 61 us; as a fallback within the split call 92).
+LISTED_TOP_K = 128
+# From this many rows on an all-greedy batch is quicker with one workgroup per row and one launch
+# (256 rows of 151,936: 31 us against 38; one row: 28 against 14).
+GREEDY_ROWS = 128
+
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 
@@ -91,6 +99,9 @@ class Sampler:
         self._param_key: tuple | None = None
         self._param_objs: tuple | None = None
         self._params: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None
+        self._top_p_rows = False  # some row of _params may be cut by top_p alone
+        self._all_greedy = False  # every row of _params takes the argmax
+        self._large_k: int | None = None  # smallest top_k of _params beyond LISTED_TOP_K
 
     def manual_seed(self, seed: int) -> None:
         self.seed = int(seed) & (2 ** 64 - 1)
@@ -117,6 +128,11 @@ class Sampler:
             host[n:2 * n] = ks.view(torch.float32)  # bit-copy the int32 top-k
             dev = host.to(device, non_blocking=True)
             self._params = (dev[:n], dev[n:2 * n].view(torch.int32), dev[2 * n:])
+            drawn = [p for p in normalized if p.temperature > 0 and p.top_p > 0]
+            self._top_p_rows = any(p.top_p < 1 and (p.top_k <= 0 or p.top_k > LISTED_TOP_K)
+                                   for p in drawn)
+            self._all_greedy = not drawn
+            self._large_k = min((p.top_k for p in drawn if p.top_k > LISTED_TOP_K), default=None)
             self._param_key = key
         return self._params
 
@@ -133,10 +149,19 @@ class Sampler:
         if rows == 0:
             return out
         temperature, top_k, top_p = self._device_params(params_list, logits.device)
-        check(lib().mi355x_sample(logits.data_ptr(), rows, logits.size(1), logits.stride(0),
-                                  _DTYPES[logits.dtype], temperature.data_ptr(),
-                                  top_k.data_ptr(), top_p.data_ptr(), self.seed, self.offset,
-                                  out.data_ptr(), stream_of(logits)), "sample")
+        args = (logits.data_ptr(), rows, logits.size(1), logits.stride(0),
+                _DTYPES[logits.dtype], temperature.data_ptr(), top_k.data_ptr(),
+                top_p.data_ptr(), self.seed, self.offset, out.data_ptr())
+        need = 0
+        if ((self._large_k is None or self._large_k >= logits.size(1))
+                and not (self._all_greedy and rows >= GREEDY_ROWS)):
+            need = lib().mi355x_sample_workspace_bytes(rows, logits.size(1), self._top_p_rows)
+        if need:
+            ws = torch.empty(need, dtype=torch.uint8, device=logits.device)
+            check(lib().mi355x_sample_split(*args, self._top_p_rows, ws.data_ptr(), need,
+                                            stream_of(logits)), "sample")
+        else:
+            check(lib().mi355x_sample(*args, stream_of(logits)), "sample")
         self.offset += 1
         return out
 

@@ -85,6 +85,11 @@ unsafe extern "C" {
     pub fn mi355x_sample(logits: *const c_void, rows: i64, vocab: i64, row_stride: i64,
         dtype: c_int, temperature: *const f32, top_k: *const i32, top_p: *const f32,
         seed: u64, offset: u64, out: *mut i64, stream: *mut c_void) -> *const c_char;
+    pub fn mi355x_sample_split(logits: *const c_void, rows: i64, vocab: i64, row_stride: i64,
+        dtype: c_int, temperature: *const f32, top_k: *const i32, top_p: *const f32,
+        seed: u64, offset: u64, out: *mut i64, top_p_rows: bool, workspace: *mut c_void,
+        workspace_bytes: i64, stream: *mut c_void) -> *const c_char;
+    pub fn mi355x_sample_workspace_bytes(rows: i64, vocab: i64, top_p_rows: bool) -> i64;
 }
 
 /// Introspection and host-side planning entries (ported tests, diagnostics); the serving

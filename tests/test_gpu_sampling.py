@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 import torch
 
+from llm_infer_rust_amd._native import lib
 from llm_infer_rust_amd.sampling import Sampler, SamplingError, SamplingParams
 from oracle import bf16 as obf
 from oracle import sampling as osamp
@@ -199,3 +200,94 @@ def test_top_k_candidate_path_edges_match_oracle(gpu, dtype, name, case, k, p):
     for r in range(rows):
         if ids[r] != want[r]:
             assert margins[r] < 1e-4, (case, k, p, r, ids[r], want[r], margins[r])
+
+
+ROW_KINDS = [sp(), sp(0.7, 50, 0.9), sp(1.0), sp(1.3, -1, 0.6), sp(0.8, 128), sp(0.5, 5, 0.3)]
+
+
+def one_workgroup_per_row(logits, params, seed, offset):
+    """mi355x_sample on the parameter arrays the sampler itself would pass."""
+    s = Sampler(seed)
+    t, k, p = s._device_params(params, logits.device)
+    out = torch.empty(logits.size(0), dtype=torch.int64, device=logits.device)
+    err = lib().mi355x_sample(logits.data_ptr(), logits.size(0), logits.size(1), logits.stride(0),
+                              {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}[logits.dtype],
+                              t.data_ptr(), k.data_ptr(), p.data_ptr(), seed, offset,
+                              out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert err is None
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,vocab", [(6, 16384), (7, 16385), (8, 18432), (21, 30001),
+                                        (40, 65539), (140, 70000), (300, 20000), (60, 151936)])
+def test_split_rows_equal_one_workgroup_per_row(gpu, dtype, rows, vocab):
+    """Nine and more segments per row, 1, 2 and 4 chunks per segment, rows that end inside a
+    chunk, every kind of row in one call. Equal ids: the two differ by the fp32 rounding of the
+    exponentials' sum only."""
+    g = torch.Generator().manual_seed(rows + vocab)
+    logits = (torch.randn(rows, vocab, generator=g) * 3).to(dtype).to(gpu)
+    params = [ROW_KINDS[i % len(ROW_KINDS)] for i in range(rows)]
+    s = Sampler(77)
+    s.offset = 3
+    got = s.sample_batch_device(logits, params)
+    assert torch.equal(got, one_workgroup_per_row(logits, params, 77, 3))
+    assert (lib().mi355x_sample_workspace_bytes(rows, vocab, True) == 0) == (vocab <= 16384)
+
+
+def test_large_top_k_takes_one_workgroup_per_row(gpu):
+    """A top_k past the lists: routed whole by the sampler, and correct inside a split call."""
+    logits = (torch.randn(6, 30000, generator=torch.Generator().manual_seed(4)) * 3).to(gpu)
+    params = [sp(0.9, 129, 0.8), sp(0.7, 50, 0.9), sp(), sp(1.0, 5000), sp(0.9, -1, 0.5), sp(1.0)]
+    want = one_workgroup_per_row(logits, params, 6, 0)
+    s = Sampler(6)
+    assert torch.equal(s.sample_batch_device(logits, params), want)
+    s.manual_seed(6)
+    s._large_k = None
+    assert torch.equal(s.sample_batch_device(logits, params), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("case", ["equal", "coarse", "few", "empty_segment", "sorted", "nan", "inf",
+                                  "all_hidden"])
+def test_split_rows_on_awkward_distributions(gpu, dtype, case):
+    """Lists that overflow (ties), fewer finite logits than k, segments without a finite logit,
+    every large logit in one segment, and invalid values in one segment only."""
+    rows, vocab = 2 * len(ROW_KINDS), 50000
+    g = torch.Generator().manual_seed(5)
+    logits = torch.randn(rows, vocab, generator=g)
+    if case == "equal":
+        logits.zero_()
+    elif case == "coarse":
+        logits = logits.round()
+    elif case == "few":
+        logits[:, 30:].fill_(float("-inf"))
+    elif case == "empty_segment":
+        logits[:, 2048:12000].fill_(float("-inf"))
+    elif case == "sorted":
+        logits = logits.sort(1).values * 4
+    elif case == "nan":
+        logits[::2, 33333] = float("nan")
+    elif case == "inf":
+        logits[::2, 33333] = float("inf")
+    else:
+        logits[:] = float("-inf")
+    logits = logits.to(dtype).to(gpu)
+    params = [ROW_KINDS[i % len(ROW_KINDS)] for i in range(rows)]
+    got = Sampler(9).sample_batch_device(logits, params)
+    assert torch.equal(got, one_workgroup_per_row(logits, params, 9, 0))
+
+
+def test_split_workspace_is_checked(gpu):
+    logits = torch.zeros(2, 20000, device=gpu)
+    need = lib().mi355x_sample_workspace_bytes(2, 20000, False)
+    assert 0 < need < lib().mi355x_sample_workspace_bytes(2, 20000, True)
+    t, k, p = Sampler(0)._device_params([sp(1.0)] * 2, gpu)
+    out = torch.empty(2, dtype=torch.int64, device=gpu)
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu)
+    args = (logits.data_ptr(), 2, 20000, 20000, 2, t.data_ptr(), k.data_ptr(), p.data_ptr(), 0, 0,
+            out.data_ptr(), False)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert b"workspace" in lib().mi355x_sample_split(*args, ws.data_ptr(), need - 1, stream)
+    assert b"workspace" in lib().mi355x_sample_split(*args, None, need, stream)
+    assert lib().mi355x_sample_split(*args, ws.data_ptr(), need, stream) is None
