@@ -59,6 +59,9 @@ constexpr int kDmaStages = 2;          // LDS ring depth
 constexpr int kDmaMaxEntries = 2048;   // page entries of one work item held in LDS
 static_assert(kDmaMaxEntries % 64 == 0, "entries are staged 64 at a time");
 constexpr float kLog2e = 1.4426950408889634f;
+// Up to this batch a merge workgroup serves one head: the grid has at least 256 workgroups
+// either way above it, and a request is cut into at most 8 chunks or so, one round of loads.
+constexpr int64_t kWideMergeRows = 32;
 
 // ---------------------------------------------------------------------------
 // Device buffer with geometric growth, matching the reference workspace rule
@@ -271,7 +274,6 @@ int64_t schedule(const int32_t* lengths, int64_t batch, int64_t workgroups, int6
                  int64_t tile, int32_t* work, int64_t capacity, int32_t* merge,
                  int64_t* share_out, int32_t* wg = nullptr, int64_t wg_capacity = 0,
                  int64_t* wgs_out = nullptr) {
-  constexpr int64_t kMinShareTokens = 128;
   constexpr int64_t kUnit = 8;  // cost units per tile
   // An item's prologue in cost units: 9/8 of a tile, as measured (per-workgroup end
   // times at configs 2 and 5 fit 2.5-2.6 us per tile + 2.4-2.9 us per item). With it,
@@ -295,7 +297,14 @@ int64_t schedule(const int32_t* lengths, int64_t batch, int64_t workgroups, int6
     tiles_of[r] = static_cast<int32_t>((lengths[r] + tile - 1) / tile);
     total += tiles_of[r];
   }
-  const int64_t min_share = std::max<int64_t>(1, kMinShareTokens / tile) * kUnit;
+  // The least a workgroup takes. The tile kernels stream a tile in ~1.3 us when the chip is not
+  // full, so a small batch is spread thin: one tile each up to kThinTiles tiles in all, two
+  // beyond, where the merge of that many more partials costs what the shorter shares give
+  // (one request at Hq 32, store + decode + merge, us: 1,337 tokens 12.4 at one tile, 12.5 at
+  // two, 21.9 at eight; 300 tokens 10.1, 11.6, 19.6; 4,000 tokens 18.0, 15.4, 21.9). The
+  // register kernel keeps 128 tokens.
+  constexpr int64_t kThinTiles = 128;
+  const int64_t min_share = (tile != kDmaTile ? 128 / tile : total <= kThinTiles ? 1 : 2) * kUnit;
   // Smallest share (cost units) whose walk needs at most `workgroups` workgroups: start
   // from the tile-only bound and add item costs until the walk fits.
   int64_t share = std::max((total * kUnit + workgroups - 1) / workgroups, min_share);
@@ -1131,21 +1140,26 @@ __global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
   }
 }
 
-// Split-KV merge: one wave per (request, q head), two dims per lane. Chunks are
-// combined with a running log2-sum-exp; the chunk loop is unrolled so the
-// partial loads of several chunks are in flight together.
-template <int DT>
+// Split-KV merge, two dims per lane: chunks are combined with a running log2-sum-exp, the
+// loads of kUnroll chunks in flight together. Bound by the latency of its rounds of loads.
+// WAVES = 1: one wave per (request, q head), four heads per workgroup. WAVES = 4: a workgroup
+// per (request, q head), wave w taking every fourth group of kUnroll chunks, joined through
+// LDS: batches of few requests are cut into up to a few hundred chunks each (one request of
+// 32,768 tokens, 256 chunks, store + decode + merge: 44.5 us against 60.6 with one wave).
+template <int DT, int WAVES>
 __global__ __launch_bounds__(256) void merge_kernel(DecodeArgs a, int32_t rows) {
+  static_assert(WAVES == 1 || WAVES == 4, "a workgroup holds four waves");
+  const int wave = threadIdx.x >> 6;
   const int req = blockIdx.x;
-  const int qh = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int qh = WAVES == 1 ? blockIdx.y * 4 + wave : blockIdx.y;
   const int lane = threadIdx.x & 63;
   if (req >= rows || qh >= a.num_q_heads) return;
   const int first = a.ints[a.o_merge + 2 * req];
   const int count = a.ints[a.o_merge + 2 * req + 1];
   if (count <= 1) return;
-  constexpr int kUnroll = 8;
+  constexpr int kUnroll = WAVES == 1 ? 8 : 16;
   float mx = -INFINITY, den = 0.f, acc0 = 0.f, acc1 = 0.f;
-  for (int c0 = 0; c0 < count; c0 += kUnroll) {
+  for (int c0 = WAVES == 1 ? 0 : wave * kUnroll; c0 < count; c0 += WAVES * kUnroll) {
     float lse[kUnroll];
     float2 v[kUnroll];
 #pragma unroll
@@ -1171,10 +1185,43 @@ __global__ __launch_bounds__(256) void merge_kernel(DecodeArgs a, int32_t rows) 
     }
     mx = m_new;
   }
+  if constexpr (WAVES > 1) {
+    __shared__ float part_m[WAVES], part_den[WAVES];
+    __shared__ float2 part_acc[WAVES][kWave];
+    if (lane == 0) {
+      part_m[wave] = mx;
+      part_den[wave] = den;
+    }
+    part_acc[wave][lane] = make_float2(acc0, acc1);
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) mx = fmaxf(mx, part_m[w]);  // wave 0 always has a chunk
+    den = acc0 = acc1 = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float wgt = __builtin_amdgcn_exp2f(part_m[w] - mx);  // 0 for a wave without chunks
+      const float2 v = part_acc[w][lane];
+      den = fmaf(wgt, part_den[w], den);
+      acc0 = fmaf(wgt, v.x, acc0);
+      acc1 = fmaf(wgt, v.y, acc1);
+    }
+  }
   const uint32_t packed = static_cast<uint32_t>(Elem<DT>::from_float(acc0 / den)) |
                           (static_cast<uint32_t>(Elem<DT>::from_float(acc1 / den)) << 16);
   *reinterpret_cast<uint32_t*>(a.out + req * a.out_stride_n + qh * a.out_stride_h + lane * 2) =
       packed;
+}
+
+template <int DT>
+void launch_merge(const DecodeArgs& a, int64_t batch, int64_t num_q_heads, hipStream_t s) {
+  const auto rows = static_cast<uint32_t>(batch);
+  const auto heads = static_cast<uint32_t>(num_q_heads);
+  if (batch <= kWideMergeRows)
+    merge_kernel<DT, 4><<<dim3(rows, heads), dim3(256), 0, s>>>(a, static_cast<int32_t>(batch));
+  else
+    merge_kernel<DT, 1><<<dim3(rows, (heads + 3) / 4), dim3(256), 0, s>>>(
+        a, static_cast<int32_t>(batch));
 }
 
 // Tokens per 16-lane group per loop trip. Override with MI355X_DECODE_U
@@ -1576,11 +1623,10 @@ extern "C" const char* mi355x_decode_run(const void* plan_ptr, const void* q, in
   if (!ok) return set_error("unsupported query group size");
   if (const char* err = launch_status("decode_kernel")) return err;
   if (p.graph || p.num_items > p.batch) {  // some request was split
-    const dim3 mgrid(static_cast<uint32_t>(batch), static_cast<uint32_t>((num_q_heads + 3) / 4));
     if (dtype == 0)
-      merge_kernel<0><<<mgrid, dim3(256), 0, s>>>(a, static_cast<int32_t>(batch));
+      launch_merge<0>(a, batch, num_q_heads, s);
     else
-      merge_kernel<1><<<mgrid, dim3(256), 0, s>>>(a, static_cast<int32_t>(batch));
+      launch_merge<1>(a, batch, num_q_heads, s);
     return launch_status("merge_kernel");
   }
   return nullptr;

@@ -272,3 +272,28 @@ def test_graph_plan_replays_dynamic_lengths_and_padded_rows(gpu, fixtures):
                                           table[:rows].cpu().numpy(), lens, page)
             assert_close(f32(out)[:rows].reshape(want.shape), want, f"rows={rows} len={length}")
             del batch
+
+
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (16, 8)])
+@pytest.mark.parametrize("rows,lo,hi", [(1, 17, 17), (1, 256, 256), (1, 257, 257), (1, 2048, 2048),
+                                        (1, 2100, 2100), (1, 9000, 9000), (3, 1, 1100),
+                                        (32, 20, 200), (33, 20, 200), (32, 1, 1500),
+                                        (33, 900, 1500)])
+def test_small_batches_spread_thin(gpu, hq, hkv, rows, lo, hi):
+    """Shares of one and two tiles (either side of 128 tiles in all), two to 256 chunks per
+    request, and both merge shapes (either side of 32 rows)."""
+    g = torch.Generator().manual_seed(rows + hi)
+    rng = np.random.default_rng(rows + hi)
+    lens, table, kc, vc, q = _random_decode_case(gpu, g, rng, rows, hq, hkv, 16, lo, hi,
+                                                 rows * (-(-hi // 16)) + 1, torch.bfloat16)
+    attn = make_backend(gpu, hq, hkv, 16)
+    cache = BaseAttention()
+    cache.bind_kv_cache(kc, vc)
+    meta = AttentionMetadata(BatchPhase.DECODE, block_table=torch.from_numpy(table).to(gpu),
+                             cache_seqlens=torch.from_numpy(lens).to(gpu))
+    batch = attn.prepare(meta, rows)
+    out = batch.forward(q, q, q, cache)
+    md = batch.plan.plan.read_metadata()
+    oplan.check_work_list(md["work"], md["merge"], lens.tolist())
+    want = oatt.decode_with_cache(f32(q), f32(kc), f32(vc), table, lens, 16)
+    assert_close(f32(out).reshape(want.shape), want, f"rows {rows} lens {lo}..{hi}")
