@@ -274,6 +274,14 @@ const char* mi355x_linear_add_rms_norm(const void* x, int64_t ldx, const void* w
                                        int64_t K, void* workspace, int64_t workspace_bytes,
                                        int32_t cus, int64_t dtype, void* stream);
 
+/* mi355x_linear_add_rms_norm for narrow rows: width N a multiple of 8 in 520..1024. */
+const char* mi355x_linear_add_rms_norm_narrow(const void* x, int64_t ldx, const void* w,
+                                              int64_t ldw, void* residual, int64_t ldr,
+                                              const void* norm_weight, double eps, void* out,
+                                              int64_t ldo, int64_t M, int64_t N, int64_t K,
+                                              void* workspace, int64_t workspace_bytes,
+                                              int32_t cus, int64_t dtype, void* stream);
+
 /* The QKV projection fused with the qk_norm -> rope -> K/V store pass that reads it
  * (decode batches): qkv[M, (Hq + 2 Hkv) * 128] = x . w^T, then mi355x_qk_norm_rope_store
  * on its q, k and v head views (token stride ldo, head stride 128) with every stage on
@@ -296,8 +304,8 @@ const char* mi355x_linear_qk_norm_rope_store(
  *   out[m, j] = round(silu(g) * u), g = round(y[m, j]), u = round(y[m, width + j]),
  * computed without writing y: equal bit for bit to mi355x_linear (unsplit, the
  * same tiling) followed by mi355x_silu_mul. K is never split, so no workspace.
- * config < 0 lets the library choose the tile shape by M (0, 6 and 7 are fused);
- * cus is accepted for the same call shape as mi355x_linear.
+ * config < 0 lets the library choose the tile shape for `cus` compute units (0, 6, 7 and 8
+ * are fused).
  * M <= 4096, K % 64 == 0, width % 4 == 0, 16-byte aligned x / w rows.
  * Replaces linear.rs:5-7 (gate_up, mlp.rs) followed by ops.rs:53-61
  * (fused_ops.cu:135-171). */

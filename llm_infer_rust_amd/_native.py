@@ -92,6 +92,10 @@ SIGNATURES: dict[str, tuple] = {
                                               c_i64, c_void_p, c_double, c_void_p, c_i64,
                                               c_i64, c_i64, c_i64, c_void_p, c_i64, c_i32,
                                               c_i64, c_void_p]),
+    "mi355x_linear_add_rms_norm_narrow": (c_char_p, [c_void_p, c_i64, c_void_p, c_i64, c_void_p,
+                                                     c_i64, c_void_p, c_double, c_void_p, c_i64,
+                                                     c_i64, c_i64, c_i64, c_void_p, c_i64, c_i32,
+                                                     c_i64, c_void_p]),
     "mi355x_linear_workspace_bytes": (c_i64, [c_i64, c_i64, c_i64, c_i32, c_i32, c_i32]),
     "mi355x_linear_noalloc": (c_char_p, [c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_i64,
                                          c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_i64,

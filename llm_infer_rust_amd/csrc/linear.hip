@@ -299,20 +299,22 @@ __global__ __launch_bounds__(256) void linear_reduce(const float* __restrict__ p
 // Fused epilogue for a projection followed by the residual RMSNorm (o_proj and down of a
 // decoder layer): y = round(sum of the split-K partials) (or y read back rounded when K is
 // not split), residual <- round(y + residual), out <- round(rms(y + residual) * weight),
-// the norm on the unrounded fp32 sum. One 256-lane workgroup per row, 8 columns per chunk,
-// chunk c + 256 j per lane and the same two-level sum of squares as the stand-alone
-// residual RMSNorm for these widths, so the results equal the two separate passes bit for
-// bit.
+// the norm on the unrounded fp32 sum. One workgroup of LANES per row (256, or one wave for
+// rows of up to 1024 columns), 8 columns per chunk, chunk c + LANES j per lane and the same sum
+// of squares as the stand-alone residual RMSNorm for these widths, so the results equal the two
+// separate passes bit for bit. Bound by latency: one round trip for the partials, one for the
+// stores.
 // SPLITS > 0: that many K splits, all partial loads (and the residual and weight loads)
 // issued before the first sum, so a row costs one memory round trip; 0: any count, read
 // split after split.
-template <int DT, int NCH, bool PARTIAL, int SPLITS>
-__global__ __launch_bounds__(256) void reduce_add_rms(const float* __restrict__ partial,
+template <int DT, int LANES, int NCH, bool PARTIAL, int SPLITS>
+__global__ __launch_bounds__(LANES) void reduce_add_rms(const float* __restrict__ partial,
                                                       int splits, uint16_t* out, int64_t ldo,
                                                       uint16_t* residual, int64_t ldr,
                                                       const uint16_t* __restrict__ weight,
                                                       int M, int N, float eps) {
   constexpr int kHeld = SPLITS > 0 ? SPLITS : 1;
+  static_assert(LANES == kWave || LANES == 4 * kWave, "one wave or four");
   __shared__ float wave_ss[4];
   const int64_t row = blockIdx.x;
   const int chunks = N >> 3;
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(256) void reduce_add_rms(const float* __restrict__ 
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
-    const int chunk = threadIdx.x + c * 256;
+    const int chunk = threadIdx.x + c * LANES;
     if (chunk >= chunks) continue;
     wraw[c] = ld128(weight + chunk * 8);
     if constexpr (PARTIAL) {
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(256) void reduce_add_rms(const float* __restrict__ 
   }
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
-    const int chunk = threadIdx.x + c * 256;
+    const int chunk = threadIdx.x + c * LANES;
     if (chunk >= chunks) continue;
     if constexpr (PARTIAL) {
       float4 lo = part[c][0][0], hi = part[c][0][1];
@@ -377,13 +379,15 @@ __global__ __launch_bounds__(256) void reduce_add_rms(const float* __restrict__ 
     for (int i = 0; i < 8; ++i) ss = fmaf(vals[c][i], vals[c][i], ss);
   }
   ss = wave_sum(ss);
-  if (threadIdx.x % kWave == 0) wave_ss[threadIdx.x / kWave] = ss;
-  __syncthreads();
-  ss = (wave_ss[0] + wave_ss[1]) + (wave_ss[2] + wave_ss[3]);
+  if constexpr (LANES > kWave) {
+    if (threadIdx.x % kWave == 0) wave_ss[threadIdx.x / kWave] = ss;
+    __syncthreads();
+    ss = (wave_ss[0] + wave_ss[1]) + (wave_ss[2] + wave_ss[3]);
+  }
   const float scale = rsqrtf(ss / static_cast<float>(N) + eps);
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
-    const int chunk = threadIdx.x + c * 256;
+    const int chunk = threadIdx.x + c * LANES;
     if (chunk < chunks) {
       float wf[8];
       unpack8<DT>(wraw[c], wf);
@@ -395,20 +399,22 @@ __global__ __launch_bounds__(256) void reduce_add_rms(const float* __restrict__ 
   }
 }
 
-template <int DT, int NCH, bool PARTIAL>
+template <int DT, int LANES, int NCH, bool PARTIAL>
 void launch_reduce_add_rms_splits(const float* partial, int splits, uint16_t* out, int64_t ldo,
                                   uint16_t* residual, int64_t ldr, const uint16_t* weight,
                                   int M, int N, float eps, hipStream_t s) {
-  const dim3 grid(static_cast<uint32_t>(M)), block(256);
+  const dim3 grid(static_cast<uint32_t>(M)), block(LANES);
 #define MI355X_REDUCE_ADD_RMS(S)                                                            \
-  reduce_add_rms<DT, NCH, PARTIAL, S><<<grid, block, 0, s>>>(partial, splits, out, ldo,    \
-                                                             residual, ldr, weight, M, N, eps)
+  reduce_add_rms<DT, LANES, NCH, PARTIAL, S><<<grid, block, 0, s>>>(                        \
+      partial, splits, out, ldo, residual, ldr, weight, M, N, eps)
   if (!PARTIAL || splits == 1)
     MI355X_REDUCE_ADD_RMS(1);
   else if (splits == 2)
     MI355X_REDUCE_ADD_RMS(2);
   else if (splits == 4)
     MI355X_REDUCE_ADD_RMS(4);
+  else if (splits == 8)
+    MI355X_REDUCE_ADD_RMS(8);
   else
     MI355X_REDUCE_ADD_RMS(0);
 #undef MI355X_REDUCE_ADD_RMS
@@ -419,15 +425,18 @@ void launch_reduce_add_rms(const float* partial, int splits, uint16_t* out, int6
                            uint16_t* residual, int64_t ldr, const uint16_t* weight, int M, int N,
                            float eps, hipStream_t s) {
   const int chunks = N / 8;
-  if (chunks <= 256)
-    launch_reduce_add_rms_splits<DT, 1, PARTIAL>(partial, splits, out, ldo, residual, ldr,
-                                                 weight, M, N, eps, s);
+  if (chunks <= 128)
+    launch_reduce_add_rms_splits<DT, kWave, 2, PARTIAL>(partial, splits, out, ldo, residual, ldr,
+                                                        weight, M, N, eps, s);
+  else if (chunks <= 256)
+    launch_reduce_add_rms_splits<DT, 256, 1, PARTIAL>(partial, splits, out, ldo, residual, ldr,
+                                                      weight, M, N, eps, s);
   else if (chunks <= 512)
-    launch_reduce_add_rms_splits<DT, 2, PARTIAL>(partial, splits, out, ldo, residual, ldr,
-                                                 weight, M, N, eps, s);
+    launch_reduce_add_rms_splits<DT, 256, 2, PARTIAL>(partial, splits, out, ldo, residual, ldr,
+                                                      weight, M, N, eps, s);
   else
-    launch_reduce_add_rms_splits<DT, 4, PARTIAL>(partial, splits, out, ldo, residual, ldr,
-                                                 weight, M, N, eps, s);
+    launch_reduce_add_rms_splits<DT, 256, 4, PARTIAL>(partial, splits, out, ldo, residual, ldr,
+                                                      weight, M, N, eps, s);
 }
 
 struct TileConfig {
@@ -444,6 +453,7 @@ constexpr TileConfig kConfigs[] = {
     {256, 64, 8, 1, 4},   // wave 32 x 64
     {128, 128, 4, 2, 3},  // wave 32 x 64, shallow ring
     {64, 128, 2, 4, 5},   // wave 32 x 32
+    {64, 64, 2, 2, 4},    // wave 32 x 32
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -472,7 +482,8 @@ void launch_dt(int config, const LinearArgs& a, int blocks, hipStream_t s) {
     case 4: launch_any<DT, 4>(a, blocks, s); break;
     case 5: launch_any<DT, 5>(a, blocks, s); break;
     case 6: launch_any<DT, 6>(a, blocks, s); break;
-    default: launch_any<DT, 7>(a, blocks, s); break;
+    case 7: launch_any<DT, 7>(a, blocks, s); break;
+    default: launch_any<DT, 8>(a, blocks, s); break;
   }
 }
 
@@ -490,6 +501,9 @@ bool launch_silu(int config, const LinearArgs& a, int blocks, hipStream_t s) {
     case 7:
       linear_kernel<DT, 64, 128, 2, 4, 5, false, true><<<dim3(blocks), dim3(512), 0, s>>>(a);
       return true;
+    case 8:
+      linear_kernel<DT, 64, 64, 2, 2, 4, false, true><<<dim3(blocks), dim3(256), 0, s>>>(a);
+      return true;
     default:
       return false;
   }
@@ -501,27 +515,56 @@ struct Choice {
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Tile shape and split count: for each tile shape in order of preference, the fewest
-// K splits that give at least 3/4 of a workgroup per CU; the first shape that needs at
-// most 4 splits wins, else the one needing the fewest. Measured on MI355X at the
-// Qwen3-8B decode shapes (M = 1..256) with the weights streamed from HBM (rotating over
-// more than 1 GB): 128 x 128 tiles with up to 4 splits beat smaller tiles with fewer
-// splits at 128-192 rows (QKV at 192 rows 27.7 us against 29.8 for 64 x 128 tiles
-// unsplit) and tie with them at 256 rows; the long-K down projection gains most.
+// Estimated time in us of a product on one tiling: a workgroup streams its x and w rows at
+// about 50 GB/s (the rate one CU's copies hold for this mix of L2 hits and HBM misses), a round
+// of workgroups per CU; the weights come at no more than 6 TB/s in all; split-K partials are
+// written, and read by the pass that follows, at about 5 TB/s; 3 us of launch and latency do
+// not depend on the choice. Within 15% of the measured times at the Qwen3-8B and -0.6B shapes,
+// 1 to 256 rows, and it picks the fastest tiling measured there or one within 1 us of it, e.g.
+// o_proj 4096 x 4096 at 64 rows 64 x 64 tiles and 4 splits (9.3 us; 64 x 128 and 8 splits
+// 10.4), QKV 6144 x 4096 at 24 rows 64 x 128 and 4 (11.0; 128 x 128 and 4: 12.9), at 256 rows
+// 128 x 128 and 2 (25.1; 64 x 128 unsplit 30.0), and for the narrow products of the small model
+// 64 x 64 (o_proj 1024 x 2048 at 45 rows 4.2 us against 6.9 with 128 x 128 tiles).
+double estimate(const TileConfig& t, int splits, int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t blocks = ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
+  const double per_block = double(t.bm + t.bn) * double(K / splits) * 2 / 50e3;
+  const double weights = double(N) * double(K) * 2 / 6e6;
+  const double partials = splits > 1 ? double(splits) * M * N * 8 / 5e6 : 0.;
+  return 3. + std::max(double(ceil_div(blocks, cus)) * per_block, weights) + partials;
+}
+
+// Partials the library may choose to write: what the allocation-free entry's scratch holds.
+constexpr int64_t kMaxPartialBytes = int64_t(32) << 20;
+
 Choice choose(int64_t M, int64_t N, int64_t K, int cus) {
-  const int order[] = {6, 0, 7};
-  const int64_t want = (3 * int64_t(cus)) / 4;
-  Choice best{-1, 1 << 30};
-  for (int c : order) {
-    const TileConfig& t = kConfigs[c];
-    const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
-    int s = 1;
-    while (s < 8 && tiles * s < want && K % (int64_t(2 * s) * kBK) == 0) s *= 2;
-    if (K % (int64_t(s) * kBK)) continue;
-    if (s <= 4) return {c, s};
-    if (s < best.splits) best = {c, s};
+  Choice best{7, 1};
+  double best_us = 1e30;
+  for (int c : {6, 7, 8})
+    for (int s = 1; s <= 8 && K % (int64_t(s) * kBK) == 0; s *= 2) {
+      if (s > 1 && int64_t(s) * M * N * 4 > kMaxPartialBytes) break;
+      const double us = estimate(kConfigs[c], s, M, N, K, cus);
+      if (us < best_us) {
+        best = {c, s};
+        best_us = us;
+      }
+    }
+  return best;
+}
+
+// The tile shape of a fused gate_up (N = 2 width columns, never split), by the same estimate:
+// 128 x 192 tiles at 256 rows and width 12288, 64 x 128 up to 64 rows (33 us there), and 64 x 64
+// where larger tiles leave most CUs without one (width 3072 at 45 rows 7.5 us against 9.7).
+int choose_silu(int64_t M, int64_t N, int64_t K, int cus) {
+  int best = 7;
+  double best_us = 1e30;
+  for (int c : {0, 6, 7, 8}) {
+    const double us = estimate(kConfigs[c], 1, M, N, K, cus);
+    if (us < best_us) {
+      best = c;
+      best_us = us;
+    }
   }
-  return best.config >= 0 ? best : Choice{7, 1};
+  return best;
 }
 
 }  // namespace
@@ -615,7 +658,7 @@ extern "C" const char* mi355x_linear(const void* x, int64_t ldx, const void* w, 
 // ---------------------------------------------------------------------------
 namespace mi355x {
 namespace {
-constexpr int64_t kLinearScratchBytes = int64_t(32) << 20;
+constexpr int64_t kLinearScratchBytes = kMaxPartialBytes;
 static __device__ __align__(256) uint8_t scratch[kLinearScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -660,16 +703,19 @@ extern "C" const char* mi355x_linear_noalloc(const void* x, int64_t ldx, const v
                     false, nullptr, static_cast<hipStream_t>(stream));
 }
 
-extern "C" const char* mi355x_linear_add_rms_norm(const void* x, int64_t ldx, const void* w,
-                                                  int64_t ldw, void* residual, int64_t ldr,
-                                                  const void* norm_weight, double eps, void* out,
-                                                  int64_t ldo, int64_t M, int64_t N, int64_t K,
-                                                  void* workspace, int64_t workspace_bytes,
-                                                  int32_t cus, int64_t dtype, void* stream) {
+namespace mi355x {
+namespace {
+const char* linear_add_rms_norm(const void* x, int64_t ldx, const void* w, int64_t ldw,
+                                void* residual, int64_t ldr, const void* norm_weight, double eps,
+                                void* out, int64_t ldo, int64_t M, int64_t N, int64_t K,
+                                void* workspace, int64_t workspace_bytes, int32_t cus,
+                                int64_t dtype, int64_t chunks_lo, int64_t chunks_hi,
+                                const char* widths, void* stream) {
   if (!residual || !norm_weight) return set_error("mi355x_linear_add_rms_norm: null pointer");
-  if (N % 8 || N / 8 <= 128 || N / 8 > 1024 || ldr < N || ldr % 8 || ldo % 8 ||
+  if (N % 8 || N / 8 < chunks_lo || N / 8 > chunks_hi || ldr < N || ldr % 8 || ldo % 8 ||
       !aligned(residual, 16) || !aligned(out, 16) || !aligned(norm_weight, 16))
-    return set_error("mi355x_linear_add_rms_norm: width must be 1032..8192 in 16-byte rows");
+    return set_error(std::string("mi355x_linear_add_rms_norm: width must be ") + widths +
+                     " in 16-byte rows");
   if (out == residual)  // the norm pass reads and writes both
     return set_error("mi355x_linear_add_rms_norm: out and residual must not alias");
   auto s = static_cast<hipStream_t>(stream);
@@ -696,6 +742,28 @@ extern "C" const char* mi355x_linear_add_rms_norm(const void* x, int64_t ldx, co
   }
   return launch_status("reduce_add_rms");
 }
+}  // namespace
+}  // namespace mi355x
+
+extern "C" const char* mi355x_linear_add_rms_norm(const void* x, int64_t ldx, const void* w,
+                                                  int64_t ldw, void* residual, int64_t ldr,
+                                                  const void* norm_weight, double eps, void* out,
+                                                  int64_t ldo, int64_t M, int64_t N, int64_t K,
+                                                  void* workspace, int64_t workspace_bytes,
+                                                  int32_t cus, int64_t dtype, void* stream) {
+  return linear_add_rms_norm(x, ldx, w, ldw, residual, ldr, norm_weight, eps, out, ldo, M, N, K,
+                             workspace, workspace_bytes, cus, dtype, 129, 1024, "1032..8192", stream);
+}
+
+extern "C" const char* mi355x_linear_add_rms_norm_narrow(const void* x, int64_t ldx, const void* w,
+                                                  int64_t ldw, void* residual, int64_t ldr,
+                                                  const void* norm_weight, double eps, void* out,
+                                                  int64_t ldo, int64_t M, int64_t N, int64_t K,
+                                                  void* workspace, int64_t workspace_bytes,
+                                                  int32_t cus, int64_t dtype, void* stream) {
+  return linear_add_rms_norm(x, ldx, w, ldw, residual, ldr, norm_weight, eps, out, ldo, M, N, K,
+                             workspace, workspace_bytes, cus, dtype, 65, 128, "520..1024", stream);
+}
 
 extern "C" const char* mi355x_linear_silu_mul(const void* x, int64_t ldx, const void* w,
                                               int64_t ldw, void* out, int64_t ldo, int64_t M,
@@ -709,10 +777,7 @@ extern "C" const char* mi355x_linear_silu_mul(const void* x, int64_t ldx, const 
     return set_error("mi355x_linear_silu_mul: unsupported shape (K % 64, width % 4, 16-byte rows)");
   if (!aligned(x, 16) || !aligned(w, 16) || !aligned(out, 8))
     return set_error("mi355x_linear_silu_mul: misaligned operand");
-  // Tile shape measured on MI355X at the Qwen3-8B gate_up shape (width 12288, K 4096):
-  // 128 x 192 tiles from 129 rows up (62.6 us at 256 rows against 66.5 for hipBLASLt plus
-  // the SiLU pass), 128 x 128 for 65..128 rows, 64 x 128 below.
-  if (config < 0) config = M > 128 ? 0 : (M > 64 ? 6 : 7);
+  if (config < 0) config = choose_silu(M, N, K, cus > 0 ? cus : 256);
   if (config >= kNumConfigs) return set_error("mi355x_linear_silu_mul: invalid tile configuration");
   const TileConfig& t = kConfigs[config];
   LinearArgs a{};

@@ -322,6 +322,19 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | Non
     return out
 
 
+def _aligned16(*tensors: torch.Tensor) -> bool:
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def uses_fused_norm_kernel(rows: int, n: int, k: int) -> bool:
+    """Whether ``linear_add_rms_norm`` runs the projection and the norm as this library's two
+    launches. Unlike ``linear`` also for few rows of a long K: the product's split-K partials
+    are summed in the norm pass, which it would need anyway (down 4096 x 12288 with its norm at
+    24 rows: 22 us against 31 on hipBLASLt and a norm launch; one row 21 against 24)."""
+    return (0 < rows <= DECODE_MAX_ROWS and n <= DECODE_MAX_N and n % 8 == 0
+            and 64 < n // 8 and k % 64 == 0)
+
+
 def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor,
                         norm_weight: torch.Tensor,
                         eps: float) -> tuple[torch.Tensor, torch.Tensor]:
@@ -332,10 +345,12 @@ def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.T
     m, k = (x.shape if x.dim() == 2 else (0, 0))
     n = weight.size(0)
     if (x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and weight.is_contiguous()
-            and uses_decode_kernel(m, n, k) and n % 8 == 0 and 128 < n // 8 <= 1024
+            and uses_fused_norm_kernel(m, n, k)
             and x.stride(0) % 8 == 0 and residual.dim() == 2 and residual.shape == (m, n)
             and residual.stride(1) == 1 and residual.dtype == x.dtype
-            and residual.device == x.device and residual.stride(0) % 8 == 0):
+            and residual.device == x.device and residual.stride(0) % 8 == 0
+            and ((n > 1024 and uses_decode_kernel(m, n, k))
+                 or _aligned16(x, weight, residual, norm_weight))):
         _require_device(x, "linear_add_rms_norm")
         dt = dtype_code(x)
         _check_weight(x, norm_weight, n)
@@ -345,7 +360,9 @@ def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.T
         cus = _native.device_cus(x.device)
         need = lib().mi355x_linear_workspace_bytes(m, n, k, cus, -1, -1)
         ws = torch.empty(max(int(need), 16), dtype=torch.uint8, device=x.device) if need else None
-        check(lib().mi355x_linear_add_rms_norm(
+        entry = (lib().mi355x_linear_add_rms_norm if n > 1024
+                 else lib().mi355x_linear_add_rms_norm_narrow)
+        check(entry(
             x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), residual.data_ptr(),
             residual.stride(0), norm_weight.data_ptr(), float(eps), out.data_ptr(), n, m, n, k,
             None if ws is None else ws.data_ptr(), int(need), cus, dt, stream_of(x)),

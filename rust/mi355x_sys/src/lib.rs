@@ -74,6 +74,10 @@ unsafe extern "C" {
         residual: *mut c_void, ldr: i64, norm_weight: *const c_void, eps: f64,
         out: *mut c_void, ldo: i64, m: i64, n: i64, k: i64, workspace: *mut c_void,
         workspace_bytes: i64, cus: i32, dtype: i64, stream: *mut c_void) -> *const c_char;
+    pub fn mi355x_linear_add_rms_norm_narrow(x: *const c_void, ldx: i64, w: *const c_void,
+        ldw: i64, residual: *mut c_void, ldr: i64, norm_weight: *const c_void, eps: f64,
+        out: *mut c_void, ldo: i64, m: i64, n: i64, k: i64, workspace: *mut c_void,
+        workspace_bytes: i64, cus: i32, dtype: i64, stream: *mut c_void) -> *const c_char;
     pub fn mi355x_linear_silu_mul(x: *const c_void, ldx: i64, w: *const c_void, ldw: i64,
         out: *mut c_void, ldo: i64, m: i64, width: i64, k: i64, cus: i32, config: i32,
         dtype: i64, stream: *mut c_void) -> *const c_char;

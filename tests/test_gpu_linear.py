@@ -213,3 +213,46 @@ def test_k_phases(gpu, m, n, k, config, splits):
     steps than phases, step counts that are no power of two, and one or several M tiles."""
     x, w = operands(m, n, k, torch.bfloat16, gpu, m + n + k)
     check_product(ops.decode_linear(x, w, config=config, splits=splits), x, w)
+
+
+@pytest.mark.parametrize("m,n,k,dtype", [(1, 4096, 12288, torch.bfloat16),
+                                         (31, 4096, 12288, torch.float16),
+                                         (45, 1024, 2048, torch.float16),
+                                         (1, 1024, 3072, torch.bfloat16),
+                                         (256, 1024, 3072, torch.bfloat16),
+                                         (7, 520, 64, torch.bfloat16),
+                                         (130, 776, 1024, torch.bfloat16)])
+def test_fused_residual_norm_of_few_rows_and_narrow_widths(gpu, m, n, k, dtype):
+    """One wave per row up to 1,024 columns, split and not, and few rows of a long K: equal to
+    decode_linear then add_rms_norm bit for bit; a misaligned norm weight takes the two steps."""
+    assert ops.uses_fused_norm_kernel(m, n, k)
+    x, w = operands(m, n, k, dtype, gpu, m * 7 + n + k)
+    g = torch.Generator().manual_seed(n + k)
+    residual = torch.randn(m, n, generator=g).to(dtype).to(gpu)
+    gamma = (torch.rand(n + 1, generator=g) + 0.5).to(dtype).to(gpu)
+    sep, fused, odd = residual.clone(), residual.clone(), residual.clone()
+    want, _ = ops.add_rms_norm(ops.decode_linear(x, w), sep, gamma[:n], 1e-6)
+    got, _ = ops.linear_add_rms_norm(x, w, fused, gamma[:n], 1e-6)
+    assert torch.equal(got, want) and torch.equal(fused, sep)
+    if n <= 1024:
+        ops.linear_add_rms_norm(x, w, odd, gamma[1:], 1e-6)
+        assert torch.equal(odd, sep)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (64, 128, 128), (65, 192, 1024), (200, 1024, 512),
+                                   (45, 4096, 1024), (33, 260, 2048)])
+@pytest.mark.parametrize("splits", [1, 2, 8])
+def test_small_tiles(gpu, m, n, k, splits):
+    """64 x 64 tiles: full and ragged in both directions, one to 16 K steps per split."""
+    if k % (64 * splits):
+        splits = 1
+    x, w = operands(m, n, k, torch.bfloat16, gpu, m + n + k)
+    check_product(ops.decode_linear(x, w, config=8, splits=splits), x, w)
+    check_product(ops.decode_linear(x, w), x, w)
+
+
+@pytest.mark.parametrize("m,width,k", [(45, 3072, 1024), (1, 196, 128), (130, 100, 512)])
+def test_small_tiles_fused_gate_up(gpu, m, width, k):
+    x, w = operands(m, 2 * width, k, torch.bfloat16, gpu, m + width)
+    two_step = ops.silu_and_mul(ops.decode_linear(x, w, config=8, splits=1))
+    assert torch.equal(ops.decode_linear_silu_mul(x, w, config=8), two_step)
