@@ -271,7 +271,7 @@ int64_t items_capacity_for(const LaunchShape& s, int64_t rows, int64_t row_token
 // wg[i] = first item of workgroup i (wg[workgroups] = item count). Returns the item
 // count, or -1 when a capacity is too small.
 int64_t schedule(const int32_t* lengths, int64_t batch, int64_t workgroups, int64_t max_item,
-                 int64_t tile, int32_t* work, int64_t capacity, int32_t* merge,
+                 int64_t tile, bool graph, int32_t* work, int64_t capacity, int32_t* merge,
                  int64_t* share_out, int32_t* wg = nullptr, int64_t wg_capacity = 0,
                  int64_t* wgs_out = nullptr) {
   constexpr int64_t kUnit = 8;  // cost units per tile
@@ -292,19 +292,24 @@ int64_t schedule(const int32_t* lengths, int64_t batch, int64_t workgroups, int6
   const int64_t max_item_tiles = std::max<int64_t>(1, max_item / tile);
   // Tiles per request, computed once (the walks below run a dozen times per plan).
   std::vector<int32_t> tiles_of(batch);
-  int64_t total = 0;
+  int64_t total = 0, longest = 0;
   for (int64_t r = 0; r < batch; ++r) {
     tiles_of[r] = static_cast<int32_t>((lengths[r] + tile - 1) / tile);
     total += tiles_of[r];
+    longest = std::max<int64_t>(longest, tiles_of[r]);
   }
   // The least a workgroup takes. The tile kernels stream a tile in ~1.3 us when the chip is not
   // full, so a small batch is spread thin: one tile each up to kThinTiles tiles in all, two
   // beyond, where the merge of that many more partials costs what the shorter shares give
   // (one request at Hq 32, store + decode + merge, us: 1,337 tokens 12.4 at one tile, 12.5 at
   // two, 21.9 at eight; 300 tokens 10.1, 11.6, 19.6; 4,000 tokens 18.0, 15.4, 21.9). The
-  // register kernel keeps 128 tokens.
+  // register kernel keeps 128 tokens, and so do eager plans of requests that short: whole, they
+  // need no merge launch, which costs an eager caller what the split gives (a graph plan
+  // launches the merge in any case).
   constexpr int64_t kThinTiles = 128;
-  const int64_t min_share = (tile != kDmaTile ? 128 / tile : total <= kThinTiles ? 1 : 2) * kUnit;
+  constexpr int64_t kWideShare = 128;  // tokens
+  const bool wide = tile != kDmaTile || (!graph && longest * tile <= kWideShare);
+  const int64_t min_share = (wide ? kWideShare / tile : total <= kThinTiles ? 1 : 2) * kUnit;
   // Smallest share (cost units) whose walk needs at most `workgroups` workgroups: start
   // from the tile-only bound and add item costs until the walk fits.
   int64_t share = std::max((total * kUnit + workgroups - 1) / workgroups, min_share);
@@ -1318,7 +1323,7 @@ extern "C" int64_t mi355x_decode_schedule(const int32_t* lengths, int64_t batch,
   // The host-only view: page size 1 and no cap on item length.
   const LaunchShape shape = launch_shape(cus, num_kv_heads, 1);
   return schedule(lengths, batch, shape.workgroups, std::numeric_limits<int32_t>::max(),
-                  shape.tile, work,
+                  shape.tile, /*graph=*/false, work,
                   work_capacity, merge, chunk_tokens);
 }
 
@@ -1462,7 +1467,7 @@ extern "C" void* mi355x_decode_prepare(void* existing, const int32_t* block_tabl
                                       (plan->host_lengths[r] + page_size - 1) / page_size);
     int64_t chunk = 0, wgs = 0;
     const int64_t items = schedule(plan->host_lengths.data(), batch, shape.workgroups,
-                                   shape.max_item, shape.tile, host + layout.o_work, items_cap,
+                                   shape.max_item, shape.tile, graph, host + layout.o_work, items_cap,
                                    host + layout.o_merge, &chunk, host + layout.o_wg, wg_cap, &wgs);
     if (items < 0) {
       set_error("decode work list exceeds its capacity");
