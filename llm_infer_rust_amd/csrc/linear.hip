@@ -3,9 +3,9 @@
 // Replaces the reference's `x.matmul(w.T)` (src/layers/linear.rs:5-7, cuBLAS through
 // tch) for the decoder layer's QKV, o_proj and down projections when the batch is a
 // decode batch (M <= 256 rows), the last two optionally fused with the residual RMSNorm
-// that follows them, and the gate_up projection fused with SiLU x mul. Prefill-sized
-// products and the lm_head stay on hipBLASLt, which runs them near the MFMA rate or at a
-// weight-streaming rate this kernel does not beat.
+// that follows them, the gate_up projection fused with SiLU x mul, and the lm_head of up to 64
+// rows. Prefill-sized products and larger heads stay on hipBLASLt, which runs them near the
+// MFMA rate.
 //
 // Why a kernel of its own: at M = 256 the four per-layer products carry 99 GFLOP
 // over 386 MB of weights, so they sit at the ridge between the MFMA rate and HBM
@@ -517,8 +517,9 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Estimated time in us of a product on one tiling: a workgroup streams its x and w rows at
 // about 50 GB/s (the rate one CU's copies hold for this mix of L2 hits and HBM misses), a round
-// of workgroups per CU; the weights come at no more than 6 TB/s in all; split-K partials are
-// written, and read by the pass that follows, at about 5 TB/s; 3 us of launch and latency do
+// of workgroups per CU; the weights come at no more than 6 TB/s in all, or 5.2 where the tile
+// does not divide N / 2 and every workgroup starts at the same K step (a 151,936-row head at
+// one row: 64 x 64 tiles 190 us, 64 x 128 tiles 235); split-K partials are written, and read by the pass that follows, at about 5 TB/s; 3 us of launch and latency do
 // not depend on the choice. Within 15% of the measured times at the Qwen3-8B and -0.6B shapes,
 // 1 to 256 rows, and it picks the fastest tiling measured there or one within 1 us of it, e.g.
 // o_proj 4096 x 4096 at 64 rows 64 x 64 tiles and 4 splits (9.3 us; 64 x 128 and 8 splits
@@ -528,7 +529,8 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 double estimate(const TileConfig& t, int splits, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t blocks = ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
   const double per_block = double(t.bm + t.bn) * double(K / splits) * 2 / 50e3;
-  const double weights = double(N) * double(K) * 2 / 6e6;
+  const double stream = (N / 2) % t.bn == 0 ? 6e6 : 5.2e6;
+  const double weights = double(N) * double(K) * 2 / stream;
   const double partials = splits > 1 ? double(splits) * M * N * 8 / 5e6 : 0.;
   return 3. + std::max(double(ceil_div(blocks, cus)) * per_block, weights) + partials;
 }

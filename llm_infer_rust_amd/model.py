@@ -14,8 +14,9 @@ Follows the reference layer sequence (``src/models/qwen3/model.rs:155-534``):
 For decode batches (at most 256 rows) the QKV, o_proj and down projections run on this
 library's projection kernel (QKV with its split-K partials summed inside the QK-norm/RoPE/
 store pass, o_proj and down fused with the residual RMSNorm that follows them) and gate_up runs
-fused with SiLU x mul; prefill-sized products and the lm_head are
-library GEMMs (torch -> hipBLASLt). Everything around them is this library's HIP code. Configuration fields and defaults follow ``src/models/qwen3/config.rs:9-42``.
+fused with SiLU x mul, as does the lm_head of up to 64 rows; prefill-sized products and larger
+heads are library GEMMs (torch -> hipBLASLt). Everything around them is this library's HIP code.
+Configuration fields and defaults follow ``src/models/qwen3/config.rs:9-42``.
 """
 from __future__ import annotations
 
@@ -201,10 +202,7 @@ class Qwen3Model:
         hidden = x
         if logits_indices is not None:
             hidden = hidden.index_select(0, logits_indices)
-        if logits_out is not None:
-            torch.matmul(hidden, self.lm_head.t(), out=logits_out)
-            return logits_out
-        return F.linear(hidden, self.lm_head)
+        return ops.head_linear(hidden, self.lm_head, logits_out)
 
 
 __all__ = ["Qwen3Config", "Qwen3Model", "Qwen3Layer"]

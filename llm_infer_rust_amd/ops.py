@@ -274,9 +274,9 @@ def linear_qk_norm_rope_store(x: torch.Tensor, weight: torch.Tensor, q_heads: in
 # columns go to the gfx950 projection kernel; long-K products (K > 4096) only from
 # DECODE_LONG_K_MIN_ROWS rows up. Everything else stays on hipBLASLt through
 # F.linear. The bounds come from timing both on MI355X at the Qwen3-8B shapes: the
-# kernel wins on QKV, o_proj and down (1.2-2.8x at 64-256 rows); hipBLASLt keeps the
-# lm_head and prefill-sized products, and gate_up goes to the fused gate_up + SiLU entry
-# (``linear_silu_mul``).
+# kernel wins on QKV, o_proj and down (1.2-2.8x at 64-256 rows); hipBLASLt keeps
+# prefill-sized products, the lm_head has a rule of its own (``head_linear``), and gate_up goes
+# to the fused gate_up + SiLU entry (``linear_silu_mul``).
 DECODE_MAX_ROWS = 256
 DECODE_MAX_N = 8192
 DECODE_LONG_K_MIN_ROWS = 32
@@ -412,6 +412,32 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return silu_and_mul(linear(x, weight))
 
 
+# The head's product (more columns than the layer products) of up to this many rows goes to the
+# gfx950 kernel: 151,936 x 4096 at 1 / 24 / 64 rows 190 / 200 / 248 us (6.5 TB/s of weights at
+# one row) against 243 / 260 / 264 on hipBLASLt, which is quicker from 96 rows (274 against
+# 280); 151,936 x 1024 50 / 54 / 67 against 60 / 72 / 79.
+HEAD_MAX_ROWS = 64
+
+
+def head_linear(x: torch.Tensor, weight: torch.Tensor,
+                out: torch.Tensor | None = None) -> torch.Tensor:
+    """``x @ weight.T`` for the lm_head (``weight [vocab, K]``), into ``out`` when given."""
+    if (x.is_cuda and x.dim() == 2 and weight.dim() == 2 and 0 < x.size(0) <= HEAD_MAX_ROWS
+            and weight.size(0) > DECODE_MAX_N and weight.size(0) % 4 == 0
+            and x.size(1) % 64 == 0 and weight.size(1) == x.size(1)
+            and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype
+            and weight.device == x.device and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and weight.is_contiguous() and _aligned16(x, weight)
+            and (out is None or (out.shape == (x.size(0), weight.size(0))
+                                 and out.dtype == x.dtype and out.device == x.device
+                                 and out.stride(1) == 1 and out.stride(0) % 4 == 0
+                                 and out.data_ptr() % 8 == 0))):
+        return decode_linear(x, weight, out=out)
+    if out is not None:
+        return torch.matmul(x, weight.t(), out=out)
+    return torch.nn.functional.linear(x, weight)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``x @ weight.T``: decode-sized products on the gfx950 kernel, the rest on
     hipBLASLt (``src/layers/linear.rs:5-7``)."""
@@ -423,6 +449,6 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 __all__ = ["rms_norm", "add_rms_norm", "qk_norm", "silu_and_mul", "linear_silu_mul",
            "HalfSplitRope", "rope", "qk_norm_rope_store", "decode_linear", "linear",
-           "linear_add_rms_norm", "decode_linear_silu_mul",
+           "head_linear", "linear_add_rms_norm", "decode_linear_silu_mul",
            "uses_decode_kernel", "NativeError",
            "_native"]

@@ -256,3 +256,19 @@ def test_small_tiles_fused_gate_up(gpu, m, width, k):
     x, w = operands(m, 2 * width, k, torch.bfloat16, gpu, m + width)
     two_step = ops.silu_and_mul(ops.decode_linear(x, w, config=8, splits=1))
     assert torch.equal(ops.decode_linear_silu_mul(x, w, config=8), two_step)
+
+
+@pytest.mark.parametrize("m", [1, 64, 65])
+@pytest.mark.parametrize("vocab,k", [(16384, 128), (10004, 1024), (151936, 192)])
+def test_head_linear(gpu, m, vocab, k):
+    """The head's product either side of the row limit, with the vocabulary ending inside a tile
+    or not, into a caller's logits and into a new tensor; a width the kernel does not take."""
+    x, w = operands(m, vocab, k, torch.bfloat16, gpu, m + vocab)
+    out = torch.zeros(m, vocab, dtype=torch.bfloat16, device=gpu)
+    assert ops.head_linear(x, w, out) is out
+    check_product(out, x, w)
+    assert torch.equal(ops.head_linear(x, w), out)
+    if m <= 64:
+        assert torch.equal(out, ops.decode_linear(x, w))
+    xo, wo = operands(m, vocab + 1, k, torch.bfloat16, gpu, 3)
+    assert torch.equal(ops.head_linear(xo, wo), F.linear(xo, wo))
