@@ -58,6 +58,12 @@ constexpr int kDmaTile = 16;           // tokens per LDS tile
 constexpr int kDmaStages = 2;          // LDS ring depth
 constexpr int kDmaMaxEntries = 2048;   // page entries of one work item held in LDS
 static_assert(kDmaMaxEntries % 64 == 0, "entries are staged 64 at a time");
+// From this many bytes of K and V in a launch its copies are non-temporal: each row is read once
+// per step, and the layers of a model together (some thirty times as much) outgrow the 256 MiB
+// Infinity Cache before the next step reads it again. Measured (store + decode + merge, us a
+// layer, plain copies against these): 1,348 MB 234 -> 209, 608 MB 114 -> 101 (6.0 TB/s), 89 MB
+// 29.4 -> 27.1, 16 MB 16.0 -> 15.0; 5.5 MB, still found in the cache, 12.4 -> 12.8.
+constexpr int64_t kOnceBytes = int64_t(8) << 20;
 constexpr float kLog2e = 1.4426950408889634f;
 // Up to this batch a merge workgroup serves one head: the grid has at least 256 workgroups
 // either way above it, and a request is cut into at most 8 chunks or so, one round of loads.
@@ -108,6 +114,7 @@ struct DeviceBuffer {
 // int32 workspace layout (device and pinned staging share it):
 //   [0]                  number of workgroups (per kv-head slice)
 //   [1]                  number of work items
+//   [2]                  1: the K/V copies are non-temporal (kOnceBytes)
 //   [4, 4+B+1)           indptr
 //   [o_work, +4*cap)     work items {request, token_begin, token_end, partial}
 //   [o_merge, +2*B)      per-request {first partial, chunk count}
@@ -775,8 +782,8 @@ struct WgRecord {
 // contiguous runs. Wave w computes kv head w of the slice from LDS exactly as
 // decode_kernel does from registers.
 // ---------------------------------------------------------------------------
-template <int DT, int G, int W, int T, int S>
-__global__ __launch_bounds__(64 * W, 1) void decode_dma_kernel(DecodeArgs a) {
+template <int DT, int G, int W, int T, int S, bool ONCE>
+__device__ __forceinline__ void decode_dma(const DecodeArgs& a, uint8_t* lds, int32_t* entries) {
   constexpr int kRow = W * 256;                 // bytes of one token's slice (K or V)
   constexpr int kHalf = T * kRow;               // K (or V) bytes of one tile
   constexpr int kStage = 2 * kHalf;
@@ -785,8 +792,6 @@ __global__ __launch_bounds__(64 * W, 1) void decode_dma_kernel(DecodeArgs a) {
   constexpr int U = T / 4;                      // tokens per 16-lane group per tile
   static_assert(kRow >= 1024 && kRow % 1024 == 0, "a copy covers part of one token row");
   static_assert(kCopies % W == 0 && U % 2 == 0, "tile shape");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[S * kStage];
-  __shared__ int32_t entries[kDmaMaxEntries];
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -837,7 +842,10 @@ __global__ __launch_bounds__(64 * W, 1) void decode_dma_kernel(DecodeArgs a) {
         }
         const uint16_t* src = (half ? vslice : kslice) + static_cast<uint64_t>(slot) * row_elems +
                               ((r * 1024) % kRow) / 2 + lane * 8;
-        copy_to_lds(src, lds_base + stage * kStage + half * kHalf + r * 1024);
+        if constexpr (ONCE)
+          copy_to_lds_nt(src, lds_base + stage * kStage + half * kHalf + r * 1024);
+        else
+          copy_to_lds(src, lds_base + stage * kStage + half * kHalf + r * 1024);
       }
     };
     // Page entries of tokens [beg, end) -> LDS (the previous item's readers are done),
@@ -922,6 +930,17 @@ __global__ __launch_bounds__(64 * W, 1) void decode_dma_kernel(DecodeArgs a) {
   }
 }
 
+template <int DT, int G, int W, int T, int S>
+__global__ __launch_bounds__(64 * W, 1) void decode_dma_kernel(DecodeArgs a) {
+  constexpr int kLds = S * 2 * T * W * 256;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
+  __shared__ int32_t entries[kDmaMaxEntries];
+  if (a.ints[2])  // uniform
+    decode_dma<DT, G, W, T, S, true>(a, lds, entries);
+  else
+    decode_dma<DT, G, W, T, S, false>(a, lds, entries);
+}
+
 // ---------------------------------------------------------------------------
 // decode_mma_kernel: decode_dma_kernel's copy pipeline with the math on the matrix
 // cores, for GQA groups of 4..16 q heads per kv head (Qwen3-8B: 4). Per 16-token tile,
@@ -967,8 +986,8 @@ __device__ __forceinline__ mma_floatx4 mma_16x16x16(const uint2& a, const uint2&
                                                  __builtin_bit_cast(mma_f16x4_t, b), c, 0, 0, 0);
 }
 
-template <int DT, int G, int W, int S>
-__global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
+template <int DT, int G, int W, int S, bool ONCE>
+__device__ __forceinline__ void decode_mma(const DecodeArgs& a, uint8_t* lds, int32_t* entries) {
   constexpr int T = 16;                         // tokens per tile = the MFMAs' 16 rows
   constexpr int kRow = W * 256;                 // bytes of one token's slice (K or V)
   constexpr int kHalf = T * kRow;               // K (or V) bytes of one tile
@@ -977,8 +996,6 @@ __global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
   constexpr int kPerWave = kCopies / W;
   static_assert(G >= 2 && G <= 16, "the q heads of a group are the MFMA columns");
   static_assert(kRow >= 1024 && kRow % 1024 == 0 && kCopies % W == 0, "tile shape");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[S * kStage];
-  __shared__ int32_t entries[kDmaMaxEntries];
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1035,7 +1052,10 @@ __global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
         const int src_chunk = (chunk & ~15) | ((chunk & 15) ^ (tile_tok & 15));
         const uint16_t* src =
             (half ? vslice : kslice) + static_cast<uint64_t>(slot) * row_elems + src_chunk * 8;
-        copy_to_lds(src, lds_base + stage * kStage + half * kHalf + r * 1024);
+        if constexpr (ONCE)
+          copy_to_lds_nt(src, lds_base + stage * kStage + half * kHalf + r * 1024);
+        else
+          copy_to_lds(src, lds_base + stage * kStage + half * kHalf + r * 1024);
       }
     };
     if (!first) __syncthreads();
@@ -1143,6 +1163,17 @@ __global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
       }
     }
   }
+}
+
+template <int DT, int G, int W, int S>
+__global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
+  constexpr int kLds = S * 2 * 16 * W * 256;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
+  __shared__ int32_t entries[kDmaMaxEntries];
+  if (a.ints[2])  // uniform
+    decode_mma<DT, G, W, S, true>(a, lds, entries);
+  else
+    decode_mma<DT, G, W, S, false>(a, lds, entries);
 }
 
 // Split-KV merge, two dims per lane: chunks are combined with a running log2-sum-exp, the
@@ -1475,6 +1506,9 @@ extern "C" void* mi355x_decode_prepare(void* existing, const int32_t* block_tabl
     }
     host[0] = static_cast<int32_t>(wgs);
     host[1] = static_cast<int32_t>(items);
+    int64_t tokens = 0;
+    for (int64_t r = 0; r < batch; ++r) tokens += plan->host_lengths[r];
+    host[2] = tokens * num_kv_heads * kHeadDim * 4 >= kOnceBytes;
     // Start records: the first item of each workgroup and the page-entry index of its
     // first token (pack_page_metadata fills the slots from the block table).
     for (int64_t w = 0; w < wgs; ++w) {

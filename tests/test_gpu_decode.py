@@ -297,3 +297,26 @@ def test_small_batches_spread_thin(gpu, hq, hkv, rows, lo, hi):
     oplan.check_work_list(md["work"], md["merge"], lens.tolist())
     want = oatt.decode_with_cache(f32(q), f32(kc), f32(vc), table, lens, 16)
     assert_close(f32(out).reshape(want.shape), want, f"rows {rows} lens {lo}..{hi}")
+
+
+def test_graph_plan_crosses_the_non_temporal_size(gpu):
+    """One graph plan re-planned at lengths whose K/V is below, just at and above 8 MiB (2,048
+    tokens of 8 kv heads): the copies' hint travels with the plan, the results do not change."""
+    g = torch.Generator().manual_seed(8)
+    rng = np.random.default_rng(8)
+    _, table, kc, vc, q = _random_decode_case(gpu, g, rng, 2, 32, 8, 16, 1600, 1600, 300,
+                                              torch.bfloat16)
+    attn = make_backend(gpu, 32, 8, 16)
+    cache = BaseAttention()
+    cache.bind_kv_cache(kc, vc)
+    lengths = torch.ones(2, dtype=torch.int32, device=gpu)
+    meta = AttentionMetadata(BatchPhase.DECODE, block_table=torch.from_numpy(table).to(gpu),
+                             cache_seqlens=lengths)
+    state = attn.prepare_decode_graph(meta)
+    batch = attn.prepare(meta, 2)
+    for lens in ([1, 1], [1023, 1024], [1024, 1024], [1600, 1500], [3, 70]):
+        lengths.copy_(torch.tensor(lens, dtype=torch.int32))
+        state.prepare_replay(DecodeHostMetadata(lens))
+        out = batch.forward(q, q, q, cache)
+        want = oatt.decode_with_cache(f32(q), f32(kc), f32(vc), table, lens, 16)
+        assert_close(f32(out).reshape(want.shape), want, f"lens {lens}")
