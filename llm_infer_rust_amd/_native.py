@@ -149,8 +149,9 @@ def last_error() -> str:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    """Handle of torch's current stream on the tensor's device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of torch's current stream on the tensor's device. The raw getter: building torch's
+    Stream object around the same handle costs 1.8 us, an eighth of a small call."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def dtype_code(t: torch.Tensor) -> int:
