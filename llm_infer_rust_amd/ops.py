@@ -421,8 +421,10 @@ HEAD_MAX_ROWS = 64
 
 def head_linear(x: torch.Tensor, weight: torch.Tensor,
                 out: torch.Tensor | None = None) -> torch.Tensor:
-    """``x @ weight.T`` for the lm_head (``weight [vocab, K]``), into ``out`` when given."""
-    if (x.is_cuda and x.dim() == 2 and weight.dim() == 2 and 0 < x.size(0) <= HEAD_MAX_ROWS
+    """``x @ weight.T`` for the lm_head (``weight [vocab, K]``), into ``out`` when given. A
+    product whose gradient is wanted stays with torch, which records it."""
+    wants_grad = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
+    if (not wants_grad and x.is_cuda and x.dim() == 2 and weight.dim() == 2 and 0 < x.size(0) <= HEAD_MAX_ROWS
             and weight.size(0) > DECODE_MAX_N and weight.size(0) % 4 == 0
             and x.size(1) % 64 == 0 and weight.size(1) == x.size(1)
             and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype

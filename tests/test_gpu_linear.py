@@ -272,3 +272,15 @@ def test_head_linear(gpu, m, vocab, k):
         assert torch.equal(out, ops.decode_linear(x, w))
     xo, wo = operands(m, vocab + 1, k, torch.bfloat16, gpu, 3)
     assert torch.equal(ops.head_linear(xo, wo), F.linear(xo, wo))
+
+
+def test_head_linear_records_gradients(gpu):
+    """A head whose gradient is wanted is recorded, whatever the row count."""
+    x, w = operands(4, 16384, 128, torch.bfloat16, gpu, 11)
+    w.requires_grad_()
+    out = ops.head_linear(x, w)
+    out.backward(torch.ones_like(out))
+    assert torch.equal(out.detach(), F.linear(x, w).detach())
+    # every row of dW is the sum of four x rows: one bf16 rounding of a sum of bf16 values
+    want = x.float().sum(0).expand_as(w)
+    assert torch.allclose(w.grad.float(), want, rtol=2 ** -7, atol=1e-6)
