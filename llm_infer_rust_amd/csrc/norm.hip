@@ -262,8 +262,8 @@ __global__ __launch_bounds__(256) void norm_vec_rows(NormArgs a) {
   }
 }
 
-// Few wide rows (decode-size batches of hidden rows): one 256-lane workgroup per
-// row so a batch of a few hundred rows still spreads over every CU. Each lane
+// Wide rows: one 256-lane workgroup per row, so a batch of a few hundred rows (decode) still
+// spreads over every CU, and a row's chain of loads is short for the large ones. Each lane
 // holds NCH 128-bit chunks; the sum of squares crosses waves through LDS.
 template <int DT, int MODE, int NCH>
 __global__ __launch_bounds__(256) void norm_row_block(NormArgs a) {
@@ -376,8 +376,16 @@ const char* dispatch(const NormArgs& a, bool vec, hipStream_t s, const char* nam
     norm_vec<DT, MODE, 16, 2><<<dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s>>>(a);
     return launch_status(name);
   }
-  // Wide rows, too few of them to give every CU four rows: a workgroup per row.
-  if (vec && chunks > 128 && chunks <= 256 * 4 && a.rows < 4 * 256 * 4) {
+  // Wide rows: a workgroup per row where there are too few of them to give every CU four rows;
+  // from 32 MiB a tensor above 2048 columns, where one wave's up to eight chunks, each stored to
+  // the residual before the next is read, are a longer chain than a workgroup's two (residual
+  // norm, 8,192 x 4,096 57.5 -> 49.0 us, 4,096 x 4,096 23.5 -> 20.4, 16,000 x 2,560 69.5 -> 59.5;
+  // RMSNorm 8,192 x 4,096 29.3 -> 25.5; below it a wave per row is as quick: 4,096 x 2,560 13.2
+  // against 13.7); and for any number of rows above 4096 columns, which a wave cannot hold
+  // (residual norm 8,192 x 5,120 element by element 148.2 us, here 62.5).
+  if (vec && chunks > 128 && chunks <= 256 * 4 &&
+      (a.rows < 4 * 256 * 4 || chunks > 512 ||
+       (chunks > 256 && a.rows * chunks >= (int64_t(1) << 21)))) {
     const dim3 grid(static_cast<uint32_t>(a.rows));
     if (chunks <= 256)
       norm_row_block<DT, MODE, 1><<<grid, dim3(256), 0, s>>>(a);

@@ -219,3 +219,26 @@ def test_norms_on_pathological_rows(gpu, dtype):
     ops.qk_norm(q, k, qw, kw, 1e-6)
     check_rel(q.reshape(-1, 128), want_q, dtype, TOL[dtype][0])
     check_rel(k.reshape(-1, 128), want_k, dtype, TOL[dtype][0])
+
+
+@pytest.mark.parametrize("rows,width", [(4095, 4096), (4096, 4096), (4101, 2056), (8160, 2056),
+                                        (8161, 2056), (4101, 4104), (4097, 8192)])
+def test_wide_rows_many(gpu, rows, width):
+    """Either side of the sizes from which wide rows take a workgroup each:
+    the residual bit for bit, the norms within one bf16 rounding of fp32 (2^-8 of the value, and
+    as much again for the fp32 sum's order)."""
+    g = torch.Generator(device=gpu).manual_seed(rows + width)
+    x = torch.empty(rows, width, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    r = torch.empty_like(x).normal_(generator=g)
+    w = torch.empty(width, device=gpu).uniform_(0.5, 1.5, generator=g).to(torch.bfloat16)
+
+    def norm(t):
+        return t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-6) * w.float()
+
+    total = x.float() + r.float()
+    want, plain = norm(total), norm(x.float())
+    got_plain = ops.rms_norm(x, w, 1e-6)
+    assert torch.allclose(got_plain.float(), plain, rtol=2 ** -7, atol=1e-6)
+    out, summed = ops.add_rms_norm(x, r, w, 1e-6)
+    assert torch.equal(summed, total.to(torch.bfloat16))
+    assert torch.allclose(out.float(), want, rtol=2 ** -7, atol=1e-6)
