@@ -229,6 +229,12 @@ __device__ __forceinline__ uint4 ld128(const void* p) {
 __device__ __forceinline__ void st128(void* p, const uint4& v) {
   *reinterpret_cast<uint4*>(p) = v;
 }
+// The load with the non-temporal hint, for data that no cache will hold until its next use.
+using Words4 = uint32_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint4 ld128_nt(const void* p) {
+  const Words4 v = __builtin_nontemporal_load(static_cast<const Words4*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 
 // The decode-batch projection launcher of linear.hip (validation, tiling, split-K). With
 // leave_partials the fp32 partials [splits][M][N] stay in `workspace` unreduced and

@@ -228,22 +228,50 @@ bool head_views_vectorisable(const HeadArgs& a) {
          aligned(a.q, 16) && aligned(a.k, 16);
 }
 
-// SiLU(gate) * up with one 128-bit chunk of gate, up and out per thread.
-template <int DT>
+// SiLU(gate) * up with one 128-bit chunk of gate, up and out per thread. Bound by HBM. ID is the
+// index type: the division by the row's chunks is done in 32 bits where the chunks can be
+// counted in them (in 64 bits it alone held the pass at 5.0 TB/s: 8,192 rows of 12,288 columns,
+// 119.6 -> 102.8 us). ONCE marks a launch whose tensors outgrow the Infinity Cache (kOnceBytes):
+// gate_up is read with non-temporal loads (102.8 -> 99.5 us). The stores stay plain: without a
+// place in the cache the pass itself is quicker (94.3 us), and the product that reads out next
+// loses more (gate_up GEMM + pass + down GEMM 1,723 us with neither hint, 1,705 with the loads,
+// 1,723 with both). Two or four chunks per thread were no faster.
+template <int DT, typename ID, bool ONCE>
 __global__ __launch_bounds__(256) void silu_mul_vec(const uint16_t* __restrict__ gate_up,
-                                                    uint16_t* __restrict__ out, int64_t tokens,
+                                                    uint16_t* __restrict__ out, ID total,
                                                     int64_t width) {
-  const int64_t chunks = width >> 3;
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (id >= tokens * chunks) return;
-  const int64_t t = id / chunks;
-  const int64_t c = (id - t * chunks) << 3;
+  const ID chunks = static_cast<ID>(width >> 3);
+  const ID id = static_cast<ID>(blockIdx.x) * 256 + threadIdx.x;
+  if (id >= total) return;
+  const ID t = id / chunks;
+  const int64_t c = static_cast<int64_t>(id - t * chunks) << 3;
+  const uint16_t* gate = gate_up + static_cast<int64_t>(t) * 2 * width + c;
   float g[8], u[8], y[8];
-  unpack8<DT>(ld128(gate_up + t * 2 * width + c), g);
-  unpack8<DT>(ld128(gate_up + t * 2 * width + width + c), u);
+  unpack8<DT>(ONCE ? ld128_nt(gate) : ld128(gate), g);
+  unpack8<DT>(ONCE ? ld128_nt(gate + width) : ld128(gate + width), u);
 #pragma unroll
   for (int i = 0; i < 8; ++i) y[i] = (g[i] / (1.f + __expf(-g[i]))) * u[i];
-  st128(out + t * width + c, pack8<DT>(y));
+  st128(out + static_cast<int64_t>(id) * 8, pack8<DT>(y));
+}
+
+// From this many bytes of gate_up and out they outgrow the 256 MiB Infinity Cache, and gate_up's
+// place in it is worth more to out. Below it the loads find gate_up there and the hint costs
+// (512 rows: 7.7 us against 8.7).
+constexpr int64_t kOnceBytes = int64_t(256) << 20;
+
+template <int DT>
+void launch_silu_vec(const uint16_t* in, uint16_t* out, int64_t tokens, int64_t width,
+                     hipStream_t s) {
+  const int64_t total = tokens * (width / 8);
+  const dim3 grid(static_cast<uint32_t>((total + 255) / 256));
+  if (total > INT32_MAX)
+    silu_mul_vec<DT, int64_t, true><<<grid, dim3(256), 0, s>>>(in, out, total, width);
+  else if (total * 48 >= kOnceBytes)
+    silu_mul_vec<DT, uint32_t, true>
+        <<<grid, dim3(256), 0, s>>>(in, out, static_cast<uint32_t>(total), width);
+  else
+    silu_mul_vec<DT, uint32_t, false>
+        <<<grid, dim3(256), 0, s>>>(in, out, static_cast<uint32_t>(total), width);
 }
 
 template <int DT>
@@ -453,12 +481,10 @@ extern "C" const char* mi355x_silu_mul(const void* gate_up, void* out, int64_t t
   const auto* in = static_cast<const uint16_t*>(gate_up);
   auto* o = static_cast<uint16_t*>(out);
   if (width % 8 == 0 && aligned(gate_up, 16) && aligned(out, 16)) {
-    const int64_t threads = tokens * (width / 8);
-    const dim3 grid(static_cast<uint32_t>((threads + 255) / 256));
     if (dtype == 0)
-      silu_mul_vec<0><<<grid, dim3(256), 0, s>>>(in, o, tokens, width);
+      launch_silu_vec<0>(in, o, tokens, width, s);
     else
-      silu_mul_vec<1><<<grid, dim3(256), 0, s>>>(in, o, tokens, width);
+      launch_silu_vec<1>(in, o, tokens, width, s);
   } else {
     const int64_t threads = tokens * width;
     const dim3 grid(static_cast<uint32_t>((threads + 255) / 256));

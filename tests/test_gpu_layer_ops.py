@@ -246,3 +246,15 @@ def test_silu_mul_matches_oracle(gpu, dtype, tokens, width):
     got = f32(out)
     assert np.abs(got - obf.round_to(want, NAME[dtype])).max() <= 0.03125
     within_one_ulp(got, want, dtype)
+
+
+@pytest.mark.parametrize("tokens,width", [(1864135, 24), (1864136, 24), (701, 65544)])
+def test_silu_mul_large_launch_equals_row_blocks(gpu, tokens, width):
+    """Either side of the size from which the pass is non-temporal, with a partly filled last
+    workgroup: the same words as the rows in smaller launches."""
+    g = torch.Generator(device=gpu).manual_seed(tokens)
+    gu = torch.empty(tokens, 2 * width, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    out = ops.silu_and_mul(gu)
+    step = tokens // 5
+    for a in range(0, tokens, step):
+        assert torch.equal(out[a:a + step], ops.silu_and_mul(gu[a:a + step]))
