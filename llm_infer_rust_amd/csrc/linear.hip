@@ -61,6 +61,7 @@ struct LinearArgs {
   int32_t M, N, K;
   int32_t splits, k_per_split;  // k_per_split is a multiple of kBK
   int32_t tiles_m, tiles_n, groups;  // groups = tiles_n * splits rounded up to 8
+  int32_t keep_weights;              // the weight copies are plain ones
 };
 
 // Swizzled position of 16-byte chunk c in tile row r: c ^ f(r) with
@@ -142,23 +143,25 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void linear_kernel(LinearArgs a) {
   // First K step of this workgroup (the others follow cyclically). With every workgroup at
   // the same step, the rows' 128-byte chunks lie a row stride apart (8 KB at K 4096) and meet
   // in a subset of the memory channels; one step apart per N tile they spread over all of
-  // them: gate_up at 24 rows 38.9 -> 32.0 us (201 MB at 6.3 TB/s). Where several M tiles
-  // re-read x from L2 the phases are eight per launch, by tile mod 8 (the XCD), so that the
-  // tiles of one XCD still read the same x chunks together: down at 256 rows 38.9 us against
-  // 40.9 with a phase per tile. The phase depends on the tile modulo half the tiles, and a
-  // SILU tile's on its pair, so gate column j, up column j and their fused tile sum K in
-  // one order; where N / 2 ends inside a tile that cannot hold and every tile starts at 0.
+  // them: gate_up 24576 x 4096 at 24 rows 41.9 -> 35.3 us, 8192 x 8192 with its norm at 24 rows
+  // 36.0 -> 29.5 and at 192 rows 51.5 -> 49.9. Where several M tiles re-read x from L2 and K is
+  // at most 4096 the phases are eight, an eighth of K apart, so that more of the tiles in flight
+  // read the same x chunks: gate_up at 256 rows 62.1 us against 64.4 with a phase per tile;
+  // at K 8192 eight phases meet again (8192 x 8192 at 192 rows 59.9 us). The phase depends on
+  // the tile modulo half the tiles, and a SILU tile's on its pair, so with the same tile shape
+  // gate column j, up column j and their fused tile sum K in one order; where N / 2 ends inside
+  // a tile that cannot hold and every tile starts at 0.
   int kt = 0;
   if ((a.N / 2) % BN == 0) {
     const int phase = SILU ? tn >> 1 : tn % (a.tiles_n >> 1);
-    kt = a.tiles_m == 1 ? phase % n_k : (phase & 7) * n_k / 8;
+    kt = a.tiles_m == 1 || a.K > 4096 ? phase % n_k : (phase & 7) * n_k / 8;
   }
-  // The weights are read once, so their copies are non-temporal and leave L2 to x (24 rows,
-  // gate_up: 44.4 -> 39.1 us before the phases above; 256 rows, QKV 28.1 -> 26.1).
+  // Weights that are read once are copied non-temporally and leave L2 to x (gate_up at 24 rows
+  // 38.8 -> 35.3 us); keep_weights is the host's word that several M tiles read them from L2.
   auto issue = [&](int stage) {
 #pragma unroll
     for (int j = 0; j < kCopies; ++j) {
-      if (8 * (wave + NW * j) < BM)
+      if (8 * (wave + NW * j) < BM || a.keep_weights)
         copy_to_lds(src[j] + kt * kBK, dst[j] + stage * kStageBytes);
       else
         copy_to_lds_nt(src[j] + kt * kBK, dst[j] + stage * kStageBytes);
@@ -535,6 +538,17 @@ double estimate(const TileConfig& t, int splits, int64_t M, int64_t N, int64_t K
   return 3. + std::max(double(ceil_div(blocks, cus)) * per_block, weights) + partials;
 }
 
+// Whether the weights' copies are plain instead of non-temporal. Several M tiles read each weight
+// tile, and L2 serves all but the first reader only while they run in step. They part where the
+// last M tile is nearly empty (its x rows are one row repeated, so it waits less): 5120 x 17408
+// with its norm at 129 / 144 / 160 rows 76 / 75 / 68 us non-temporal, 63 / 66 / 69 plain, 4096 x
+// 12288 at 72 rows 33.3 and 30.8. Up to 32 MiB of weights plain copies are quicker for any last
+// tile (4096 x 4096 at 192 rows 22.5 and 21.1); above it they cost (8192 x 8192 at 224 rows 51.9
+// and 54.4, 4096 x 12288 at 208 rows 41.7 and 43.7).
+bool keeps_weights(const TileConfig& t, int64_t M, int64_t N, int64_t K) {
+  return M > t.bm && ((M - 1) % t.bm < t.bm / 4 || N * K * 2 <= (int64_t(32) << 20));
+}
+
 // Partials the library may choose to write: what the allocation-free entry's scratch holds.
 constexpr int64_t kMaxPartialBytes = int64_t(32) << 20;
 
@@ -620,6 +634,7 @@ const char* run_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, v
   a.tiles_m = static_cast<int32_t>(ceil_div(M, t.bm));
   a.tiles_n = static_cast<int32_t>(ceil_div(N, t.bn));
   a.groups = static_cast<int32_t>(ceil_div(int64_t(a.tiles_n) * a.splits, 8) * 8);
+  a.keep_weights = keeps_weights(t, M, N, K);
   const int64_t blocks = int64_t(a.groups) * a.tiles_m;
   if (blocks > (int64_t(1) << 31) - 1) return set_error("mi355x_linear: grid too large");
   if (dtype == 0)
@@ -797,6 +812,7 @@ extern "C" const char* mi355x_linear_silu_mul(const void* x, int64_t ldx, const 
   a.tiles_m = static_cast<int32_t>(ceil_div(M, t.bm));
   a.tiles_n = static_cast<int32_t>(ceil_div(N, t.bn));
   a.groups = static_cast<int32_t>(ceil_div(a.tiles_n, 8) * 8);
+  a.keep_weights = keeps_weights(t, M, N, K);
   const int64_t blocks = int64_t(a.groups) * a.tiles_m;
   if (blocks > (int64_t(1) << 31) - 1) return set_error("mi355x_linear_silu_mul: grid too large");
   auto s = static_cast<hipStream_t>(stream);

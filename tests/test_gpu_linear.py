@@ -215,6 +215,18 @@ def test_k_phases(gpu, m, n, k, config, splits):
     check_product(ops.decode_linear(x, w, config=config, splits=splits), x, w)
 
 
+@pytest.mark.parametrize("m", [33, 64, 65, 80, 81, 128, 129, 160, 161])
+@pytest.mark.parametrize("n,k", [(512, 4160), (512, 4096), (4224, 4096)])
+@pytest.mark.parametrize("config", [6, 7, 8])
+def test_weights_read_by_several_row_tiles(gpu, m, n, k, config):
+    """Last row tiles up to a quarter full and just past it, weights up to 32 MiB and just past it,
+    a K step of its own for every column tile (K past 4096) and eight of them."""
+    x, w = operands(m, n, k, torch.bfloat16, gpu, m + n + k)
+    check_product(ops.decode_linear(x, w, config=config, splits=1), x, w)
+    two_step = ops.silu_and_mul(ops.decode_linear(x, w, config=config, splits=1))
+    assert torch.equal(ops.decode_linear_silu_mul(x, w, config=config), two_step)
+
+
 @pytest.mark.parametrize("m,n,k,dtype", [(1, 4096, 12288, torch.bfloat16),
                                          (31, 4096, 12288, torch.float16),
                                          (45, 1024, 2048, torch.float16),
