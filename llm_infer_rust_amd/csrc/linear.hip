@@ -26,6 +26,7 @@
 //   * workgroups that share a weight tile (different M tiles of it) are placed on the
 //     same XCD (workgroup i runs on XCD i mod 8), so the tile is fetched from HBM once.
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <cstdint>
 
@@ -518,24 +519,35 @@ struct Choice {
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Estimated time in us of a product on one tiling: a workgroup streams its x and w rows at
-// about 50 GB/s (the rate one CU's copies hold for this mix of L2 hits and HBM misses), a round
-// of workgroups per CU; the weights come at no more than 6 TB/s in all, or 5.2 where the tile
-// does not divide N / 2 and every workgroup starts at the same K step (a 151,936-row head at
-// one row: 64 x 64 tiles 190 us, 64 x 128 tiles 235); split-K partials are written, and read by the pass that follows, at about 5 TB/s; 3 us of launch and latency do
-// not depend on the choice. Within 15% of the measured times at the Qwen3-8B and -0.6B shapes,
-// 1 to 256 rows, and it picks the fastest tiling measured there or one within 1 us of it, e.g.
-// o_proj 4096 x 4096 at 64 rows 64 x 64 tiles and 4 splits (9.3 us; 64 x 128 and 8 splits
-// 10.4), QKV 6144 x 4096 at 24 rows 64 x 128 and 4 (11.0; 128 x 128 and 4: 12.9), at 256 rows
-// 128 x 128 and 2 (25.1; 64 x 128 unsplit 30.0), and for the narrow products of the small model
-// 64 x 64 (o_proj 1024 x 2048 at 45 rows 4.2 us against 6.9 with 128 x 128 tiles).
+// Estimated time in us of a product on one tiling. A workgroup streams its x and w rows at about
+// 50 GB/s (the rate one CU's copies hold for this mix of L2 hits and HBM misses), a round of
+// workgroups per CU; past three rounds they no longer step together. The weights come at no more
+// than 6.5 TB/s in all, or 5.4 where K is a power of two and the tile does not divide N / 2, so
+// that every workgroup starts at the same K step of rows a power of two apart (the head of 151,936
+// rows at one row: K 4096 64 x 64 tiles 192 us, 64 x 128 tiles 235; K 5120 239 and 236); each
+// further M tile takes part of that again from L2. x is re-read per N tile at about 80 TB/s, which
+// tells tile widths apart under a large head. Split-K partials are written, and read by the pass that
+// follows, at about 4.2 TB/s, with 0.6 us and 0.3 per split besides. 3 us of launch and latency do
+// not depend on the choice.
+// Fitted to every tiling of 25 shapes (hidden 1024 to 8192, K 576 to 18944) at 18 row counts from
+// 1 to 256, alone and with the norm pass, and of 23 heads at up to 64 rows: the tiling it picks
+// takes 0.5% longer than the fastest measured on average and 16% at worst, and its own figure is
+// 8% off on average, a third at worst (8192 x 1024 at 128 rows, 8.7 us for 13.7). For instance
+// o_proj 4096 x 4096 at 65 rows 64 x 128 tiles and 4 splits (15.4 us; 128 x 128 and 8 splits 16.9),
+// and the head of K 2048 at one row unsplit (104 us; 2 splits 136).
 double estimate(const TileConfig& t, int splits, int64_t M, int64_t N, int64_t K, int cus) {
-  const int64_t blocks = ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
-  const double per_block = double(t.bm + t.bn) * double(K / splits) * 2 / 50e3;
-  const double stream = (N / 2) % t.bn == 0 ? 6e6 : 5.2e6;
-  const double weights = double(N) * double(K) * 2 / stream;
-  const double partials = splits > 1 ? double(splits) * M * N * 8 / 5e6 : 0.;
-  return 3. + std::max(double(ceil_div(blocks, cus)) * per_block, weights) + partials;
+  const int64_t tiles_m = ceil_div(M, t.bm);
+  const int64_t blocks = tiles_m * ceil_div(N, t.bn) * splits;
+  const double k_bytes = double(K / splits) * 2;
+  const double per_cu = double(blocks) / cus;
+  const double rounds = per_cu < 2.85 ? std::ceil(per_cu) : per_cu + 0.23;
+  const double stream = (N / 2) % t.bn == 0 || (K & (K - 1)) != 0 ? 6.5e6 : 5.4e6;
+  const double weights = double(N) * double(K) * 2 / stream * (1. + 0.6 * double(tiles_m - 1));
+  const double x_reads = double(blocks) * double(std::min<int64_t>(M, t.bm)) * k_bytes / 80e6;
+  const double partials =
+      splits > 1 ? double(splits) * double(M) * double(N) * 8 / 4.2e6 + 0.6 + 0.3 * splits : 0.;
+  return 3. + std::max(rounds * double(t.bm + t.bn) * k_bytes / 50e3, weights) + x_reads +
+         partials;
 }
 
 // Whether the weights' copies are plain instead of non-temporal. Several M tiles read each weight
@@ -552,24 +564,34 @@ bool keeps_weights(const TileConfig& t, int64_t M, int64_t N, int64_t K) {
 // Partials the library may choose to write: what the allocation-free entry's scratch holds.
 constexpr int64_t kMaxPartialBytes = int64_t(32) << 20;
 
+// The tiling with the least estimate. K is split further only while the tiles leave less than two
+// rounds of workgroups, and 128 x 192 tiles keep 16 K steps (with fewer, filling their three
+// stages is not worth it: QKV 6144 x 2560 at 144 rows 22.3 us with 128 x 128 tiles and 2 splits,
+// 23.5 with 128 x 192 and 4).
 Choice choose(int64_t M, int64_t N, int64_t K, int cus) {
   Choice best{7, 1};
   double best_us = 1e30;
-  for (int c : {6, 7, 8})
+  for (int c : {0, 6, 7, 8}) {
+    const TileConfig& t = kConfigs[c];
+    const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
     for (int s = 1; s <= 8 && K % (int64_t(s) * kBK) == 0; s *= 2) {
-      if (s > 1 && int64_t(s) * M * N * 4 > kMaxPartialBytes) break;
-      const double us = estimate(kConfigs[c], s, M, N, K, cus);
+      if (s > 1 && (int64_t(s) * M * N * 4 > kMaxPartialBytes || tiles * s >= 4 * int64_t(cus)))
+        break;
+      if (c == 0 && K / s < 16 * kBK) break;
+      const double us = estimate(t, s, M, N, K, cus);
       if (us < best_us) {
         best = {c, s};
         best_us = us;
       }
     }
+  }
   return best;
 }
 
 // The tile shape of a fused gate_up (N = 2 width columns, never split), by the same estimate:
-// 128 x 192 tiles at 256 rows and width 12288, 64 x 128 up to 64 rows (33 us there), and 64 x 64
-// where larger tiles leave most CUs without one (width 3072 at 45 rows 7.5 us against 9.7).
+// 128 x 192 tiles at 256 rows and width 12288, 64 x 128 up to 64 rows, and 64 x 64 where larger
+// tiles leave most CUs without one (width 3072 at 45 rows 7.5 us against 9.7). The fastest of the
+// four at each of 11 widths and 18 row counts measured.
 int choose_silu(int64_t M, int64_t N, int64_t K, int cus) {
   int best = 7;
   double best_us = 1e30;

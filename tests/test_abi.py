@@ -132,6 +132,16 @@ def test_linear_workspace_bytes_query(native):
     assert f(256, 4096, 12288, 256, -1, -1) > 0
 
 
+@pytest.mark.parametrize("m,n,k,splits", [(65, 4096, 4096, 4), (96, 3072, 3072, 4),
+                                          (1, 151936, 2048, 1), (8, 151936, 4096, 1),
+                                          (144, 6144, 2560, 2)])
+def test_linear_splits_no_more_than_pays(native, m, n, k, splits):
+    """K splits where more of them were measured slower on 256 compute units (the head of 151,936
+    rows and K 2048 at one row: 104 us unsplit, 136 with two)."""
+    need = native.lib().mi355x_linear_workspace_bytes(m, n, k, 256, -1, -1)
+    assert need == (splits * m * n * 4 if splits > 1 else 0)
+
+
 @pytest.mark.parametrize("ragged", [False, True])
 @pytest.mark.parametrize("seed", range(5))
 def test_prefill_schedule_covers_every_query_block_once(native, seed, ragged):
