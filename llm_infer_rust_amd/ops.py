@@ -350,7 +350,8 @@ def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.T
             and residual.stride(1) == 1 and residual.dtype == x.dtype
             and residual.device == x.device and residual.stride(0) % 8 == 0
             and ((n > 1024 and uses_decode_kernel(m, n, k))
-                 or _aligned16(x, weight, residual, norm_weight))):
+                 or (weight.dim() == 2 and x.stride(0) >= k and residual.stride(0) >= n
+                     and _aligned16(x, weight, residual, norm_weight)))):
         _require_device(x, "linear_add_rms_norm")
         dt = dtype_code(x)
         _check_weight(x, norm_weight, n)
@@ -433,15 +434,17 @@ def head_linear(x: torch.Tensor, weight: torch.Tensor,
     """``x @ weight.T`` for the lm_head (``weight [vocab, K]``), into ``out`` when given. A
     product whose gradient is wanted stays with torch, which records it."""
     wants_grad = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
-    if (not wants_grad and x.is_cuda and x.dim() == 2 and weight.dim() == 2 and 0 < x.size(0) <= _head_rows(x.size(1))
+    if (not wants_grad and x.is_cuda and x.dim() == 2 and weight.dim() == 2
+            and 0 < x.size(0) <= _head_rows(x.size(1))
             and weight.size(0) > DECODE_MAX_N and weight.size(0) % 4 == 0
-            and x.size(1) % 64 == 0 and weight.size(1) == x.size(1)
+            and x.size(1) > 0 and x.size(1) % 64 == 0 and weight.size(1) == x.size(1)
             and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype
             and weight.device == x.device and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and weight.is_contiguous() and _aligned16(x, weight)
+            and x.stride(0) >= x.size(1) and weight.is_contiguous() and _aligned16(x, weight)
             and (out is None or (out.shape == (x.size(0), weight.size(0))
                                  and out.dtype == x.dtype and out.device == x.device
                                  and out.stride(1) == 1 and out.stride(0) % 4 == 0
+                                 and out.stride(0) >= weight.size(0)
                                  and out.data_ptr() % 8 == 0))):
         return decode_linear(x, weight, out=out)
     if out is not None:

@@ -296,3 +296,38 @@ def test_head_linear_records_gradients(gpu):
     # every row of dW is the sum of four x rows: one bf16 rounding of a sum of bf16 values
     want = x.float().sum(0).expand_as(w)
     assert torch.allclose(w.grad.float(), want, rtol=2 ** -7, atol=1e-6)
+
+
+@pytest.mark.parametrize("m", [1, 4])
+def test_fused_residual_norm_of_repeated_rows(gpu, m):
+    """Rows of stride 0, which the kernel does not read, take the two steps. Either side rounds
+    the product and the norm to bf16: within 2^-7 each."""
+    row, w = operands(1, 4096, 12288, torch.bfloat16, gpu, m)
+    x = row[0].expand(m, 12288)
+    gamma = torch.ones(4096, dtype=torch.bfloat16, device=gpu)
+    residual, want_r = (torch.zeros(m, 4096, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    want, _ = ops.add_rms_norm(F.linear(x.contiguous(), w), want_r, gamma, 1e-6)
+    got, _ = ops.linear_add_rms_norm(x, w, residual, gamma, 1e-6)
+    assert torch.allclose(got.float(), want.float(), rtol=2 ** -6, atol=1e-4)
+    assert torch.allclose(residual.float(), want_r.float(), rtol=2 ** -6, atol=1e-4)
+
+
+def test_fused_residual_norm_of_a_one_row_residual_of_stride_0(gpu):
+    x, w = operands(1, 520, 128, torch.bfloat16, gpu, 520)
+    gamma = torch.ones(520, dtype=torch.bfloat16, device=gpu)
+    want_r = torch.zeros(1, 520, dtype=torch.bfloat16, device=gpu)
+    want, _ = ops.add_rms_norm(ops.decode_linear(x, w), want_r, gamma, 1e-6)
+    residual = torch.zeros(520, dtype=torch.bfloat16, device=gpu).expand(1, 520)
+    got, _ = ops.linear_add_rms_norm(x, w, residual, gamma, 1e-6)
+    assert torch.equal(got, want) and torch.equal(residual, want_r)
+
+
+def test_head_linear_of_repeated_rows_and_empty_ones(gpu):
+    row, w = operands(1, 16384, 128, torch.bfloat16, gpu, 3)
+    x = row[0].expand(3, 128)
+    check_product(ops.head_linear(x, w), x, w)
+    out = torch.zeros(16384, dtype=torch.bfloat16, device=gpu).expand(1, 16384)
+    assert ops.head_linear(row, w, out) is out
+    check_product(out, row, w)
+    empty = ops.head_linear(row[:, :0], w[:, :0].contiguous())
+    assert empty.shape == (1, 16384) and not bool(empty.any())
