@@ -326,6 +326,18 @@ def _aligned16(*tensors: torch.Tensor) -> bool:
     return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
+def _ordinary(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may read the tensors' memory in place of a torch call that they used to
+    reach: strided, of no class or mode that takes torch's calls over, outside vmap, forward-mode
+    differentiation and tracing."""
+    return (all(t.layout == torch.strided for t in tensors)
+            and not torch.overrides.has_torch_function(tensors)
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._functorch.maybe_current_level() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._get_tracing_state() is None)
+
+
 def uses_fused_norm_kernel(rows: int, n: int, k: int) -> bool:
     """Whether ``linear_add_rms_norm`` runs the projection and the norm as this library's two
     launches. Unlike ``linear`` also for few rows of a long K: the product's split-K partials
@@ -351,7 +363,8 @@ def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.T
             and residual.device == x.device and residual.stride(0) % 8 == 0
             and ((n > 1024 and uses_decode_kernel(m, n, k))
                  or (weight.dim() == 2 and x.stride(0) >= k and residual.stride(0) >= n
-                     and _aligned16(x, weight, residual, norm_weight)))):
+                     and _aligned16(x, weight, residual, norm_weight)
+                     and _ordinary(x, weight)))):
         _require_device(x, "linear_add_rms_norm")
         dt = dtype_code(x)
         _check_weight(x, norm_weight, n)
@@ -432,9 +445,11 @@ def _head_rows(k: int) -> int:
 def head_linear(x: torch.Tensor, weight: torch.Tensor,
                 out: torch.Tensor | None = None) -> torch.Tensor:
     """``x @ weight.T`` for the lm_head (``weight [vocab, K]``), into ``out`` when given. A
-    product whose gradient is wanted stays with torch, which records it."""
-    wants_grad = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
-    if (not wants_grad and x.is_cuda and x.dim() == 2 and weight.dim() == 2
+    product whose gradient or tangent is wanted stays with torch, which records it."""
+    wants_grad = torch.is_grad_enabled() and (
+        x.requires_grad or weight.requires_grad or (out is not None and out.requires_grad))
+    if (not wants_grad and _ordinary(x, weight) and x.is_cuda and x.dim() == 2
+            and weight.dim() == 2
             and 0 < x.size(0) <= _head_rows(x.size(1))
             and weight.size(0) > DECODE_MAX_N and weight.size(0) % 4 == 0
             and x.size(1) > 0 and x.size(1) % 64 == 0 and weight.size(1) == x.size(1)

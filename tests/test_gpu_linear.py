@@ -331,3 +331,25 @@ def test_head_linear_of_repeated_rows_and_empty_ones(gpu):
     check_product(out, row, w)
     empty = ops.head_linear(row[:, :0], w[:, :0].contiguous())
     assert empty.shape == (1, 16384) and not bool(empty.any())
+
+
+def test_head_linear_keeps_torch_transforms(gpu):
+    """Forward-mode differentiation, vmap, a dispatch mode and an output that wants a gradient
+    see torch's product, as they did before the head had a kernel."""
+    x, w = operands(4, 16384, 128, torch.bfloat16, gpu, 21)
+    t = operands(4, 16384, 128, torch.bfloat16, gpu, 22)[0]
+    with torch.autograd.forward_ad.dual_level():
+        out = ops.head_linear(torch.autograd.forward_ad.make_dual(x, t), w)
+        tangent = torch.autograd.forward_ad.unpack_dual(out).tangent
+    assert tangent is not None
+    check_product(tangent, t, w)
+    scaled = torch.func.vmap(lambda s: ops.head_linear(x * s, w))(
+        torch.tensor([1.0, 2.0], dtype=torch.bfloat16, device=gpu))
+    check_product(scaled[1], x * 2, w)
+    from torch.utils.flop_counter import FlopCounterMode
+    with FlopCounterMode(display=False) as flops:
+        ops.head_linear(x, w)
+    assert flops.get_total_flops() == 2 * 4 * 16384 * 128
+    out = torch.zeros(4, 16384, dtype=torch.bfloat16, device=gpu, requires_grad=True)
+    with pytest.raises(RuntimeError):
+        ops.head_linear(x, w, out)
