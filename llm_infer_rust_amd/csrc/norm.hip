@@ -377,15 +377,16 @@ const char* dispatch(const NormArgs& a, bool vec, hipStream_t s, const char* nam
     return launch_status(name);
   }
   // Wide rows: a workgroup per row where there are too few of them to give every CU four rows;
-  // from 32 MiB a tensor above 2048 columns, where one wave's up to eight chunks, each stored to
+  // from 32 MiB a tensor and 2176 columns, where one wave's up to eight chunks, each stored to
   // the residual before the next is read, are a longer chain than a workgroup's two (residual
-  // norm, 8,192 x 4,096 57.5 -> 49.0 us, 4,096 x 4,096 23.5 -> 20.4, 16,000 x 2,560 69.5 -> 59.5;
-  // RMSNorm 8,192 x 4,096 29.3 -> 25.5; below it a wave per row is as quick: 4,096 x 2,560 13.2
-  // against 13.7); and for any number of rows above 4096 columns, which a wave cannot hold
-  // (residual norm 8,192 x 5,120 element by element 148.2 us, here 62.5).
+  // norm, 12,000 x 4,096 58.8 -> 57.1 us, 5,000 x 4,096 28.4 -> 25.4, 40,000 x 2,560 158 -> 141;
+  // RMSNorm 8,192 x 4,096 23.3 -> 21.6; below it a wave per row is as quick, and with a second
+  // chunk for a few lanes only it is quicker: residual norm 8,192 x 2,056 23.1 against 27.6); and
+  // for any number of rows above 4096 columns, which a wave cannot hold (residual norm
+  // 8,192 x 5,120 element by element 89.0 us, here 50.2).
   if (vec && chunks > 128 && chunks <= 256 * 4 &&
       (a.rows < 4 * 256 * 4 || chunks > 512 ||
-       (chunks > 256 && a.rows * chunks >= (int64_t(1) << 21)))) {
+       (chunks >= 272 && a.rows * chunks >= (int64_t(1) << 21)))) {
     const dim3 grid(static_cast<uint32_t>(a.rows));
     if (chunks <= 256)
       norm_row_block<DT, MODE, 1><<<grid, dim3(256), 0, s>>>(a);

@@ -222,7 +222,8 @@ def test_norms_on_pathological_rows(gpu, dtype):
 
 
 @pytest.mark.parametrize("rows,width", [(4095, 4096), (4096, 4096), (4101, 2056), (8160, 2056),
-                                        (8161, 2056), (4101, 4104), (4097, 8192)])
+                                        (8161, 2056), (8000, 2168), (7710, 2176),
+                                        (7711, 2176), (4101, 4104), (4097, 8192)])
 def test_wide_rows_many(gpu, rows, width):
     """Either side of the sizes from which wide rows take a workgroup each:
     the residual bit for bit, the norms within one bf16 rounding of fp32 (2^-8 of the value, and
