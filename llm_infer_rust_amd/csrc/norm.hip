@@ -383,8 +383,9 @@ const char* dispatch(const NormArgs& a, bool vec, hipStream_t s, const char* nam
   // RMSNorm 8,192 x 4,096 23.3 -> 21.6; below it a wave per row is as quick, and with a second
   // chunk for a few lanes only it is quicker: residual norm 8,192 x 2,056 23.1 against 27.6); and
   // for any number of rows above 4096 columns, which a wave cannot hold (residual norm
-  // 8,192 x 5,120 element by element 89.0 us, here 50.2).
-  if (vec && chunks > 128 && chunks <= 256 * 4 &&
+  // 8,192 x 5,120 element by element 89.0 us, here 50.2). A launch holds fewer than 2^32 threads,
+  // so 2^24 rows and more take a wave each.
+  if (vec && chunks > 128 && chunks <= 256 * 4 && a.rows < (int64_t(1) << 24) &&
       (a.rows < 4 * 256 * 4 || chunks > 512 ||
        (chunks >= 272 && a.rows * chunks >= (int64_t(1) << 21)))) {
     const dim3 grid(static_cast<uint32_t>(a.rows));

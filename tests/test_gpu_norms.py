@@ -243,3 +243,16 @@ def test_wide_rows_many(gpu, rows, width):
     out, summed = ops.add_rms_norm(x, r, w, 1e-6)
     assert torch.equal(summed, total.to(torch.bfloat16))
     assert torch.allclose(out.float(), want, rtol=2 ** -7, atol=1e-6)
+
+
+def test_more_wide_rows_than_a_launch_has_workgroups(gpu):
+    """2^24 rows of 2,176 columns (one row repeated): a workgroup each would be 2^32 threads."""
+    g = torch.Generator(device=gpu).manual_seed(24)
+    row = torch.empty(1, 2176, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    w = torch.empty(2176, device=gpu).uniform_(0.5, 1.5, generator=g).to(torch.bfloat16)
+    want = ops.rms_norm(row, w, 1e-6)[0]
+    out = ops.rms_norm(row.expand(2 ** 24, 2176), w, 1e-6)
+    for i in (0, 1, 2 ** 23, 2 ** 24 - 2, 2 ** 24 - 1):
+        assert torch.allclose(out[i].float(), want.float(), rtol=2 ** -7, atol=1e-6)
+    del out
+    torch.cuda.empty_cache()
