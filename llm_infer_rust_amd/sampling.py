@@ -118,7 +118,6 @@ class Sampler:
             return self._params
         normalized = [p.normalized() for p in params_list]
         key = (device, tuple((p.temperature, p.top_k, p.top_p) for p in normalized))
-        self._param_objs = tuple(params_list)
         if key != self._param_key:
             n = len(normalized)
             host = torch.empty(3 * n, dtype=torch.float32, pin_memory=True)
@@ -134,6 +133,7 @@ class Sampler:
             self._all_greedy = not drawn
             self._large_k = min((p.top_k for p in drawn if p.top_k > LISTED_TOP_K), default=None)
             self._param_key = key
+        self._param_objs = tuple(params_list)  # last: a build that raised is not taken for built
         return self._params
 
     def sample_batch_device(self, logits: torch.Tensor, params_list, *,
