@@ -624,7 +624,10 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
 //                    cutoff on p);
 //   race_segments    those rows' race over the survivors, per segment;
 //   sample_finish    one workgroup per row joins the segments. Rows whose lists overflow (heavy
-//                    ties) or whose parameters fit none of the above take sample_row.
+//                    ties) or whose parameters fit none of the above take sample_row. Rows with
+//                    fewer than k finite logits (a grammar's mask) and rows whose k-th p has no
+//                    fixed-point mass (sharp logits) are joined too: 5 rows of 151,936 with 30
+//                    tokens allowed 95 -> 21 us, with logits of deviation 25 286 -> 25.
 // Cutoffs and draws are sample_row's: masses are the same fixed-point sums, the race is the
 // same, and the sum of exp differs by its fp32 rounding only.
 // ---------------------------------------------------------------------------
@@ -1266,7 +1269,7 @@ __device__ bool finish_wave(const SampleArgs& a, int64_t row, const uint32_t* ca
     }
   reached = __any(reached);
   p_k = wave_max(p_k);
-  if (p_k < 0.f || (use_p && fixed_mass(p_k) == 0)) return false;
+  if (p_k < 0.f) return false;
   float s_k = INFINITY;  // the lowest s that has it
 #pragma unroll
   for (int t = 0; t < R; ++t)
@@ -1279,6 +1282,14 @@ __device__ bool finish_wave(const SampleArgs& a, int64_t row, const uint32_t* ca
     for (int t = 0; t < R; ++t)
       if (p[t] > cut && mass[t] >= mass_target(top_p)) cut = p[t];
     cut = wave_max(cut);
+  } else if (use_p && fixed_mass(p_k) == 0) {
+    // Rounding kept the whole mass below the target, and all of it lies above p_k: the cutoff is
+    // the lowest p that has any.
+    float low = INFINITY;
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      if (fx[t]) low = fminf(low, p[t]);
+    cut = -wave_max(-low);
   }
   float best = -INFINITY;
   uint32_t best_i = static_cast<uint32_t>(a.vocab);
@@ -1367,7 +1378,7 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
   // into the same words) and loads its tokens; meanwhile one wave takes a lower bound of the
   // k-th largest s from the segments' peaks, folded into 256 groups. The tokens that reach the
   // bound, little more than k, are kept for finish_candidates' work.
-  const uint32_t k = static_cast<uint32_t>(r.top_k);
+  uint32_t k = static_cast<uint32_t>(r.top_k);
   uint32_t total = 0;
   bool full = false;
   for (int j0 = 0; j0 < n; j0 += kWave) {
@@ -1383,8 +1394,11 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     if (j < n) sh.offset[j] = total + incl - c;
     total += __shfl(incl, kWave - 1);
   }
-  bool ok = !__any(full) && total >= k && total <= kRowList;  // the same in every wave
+  bool ok = !__any(full) && total <= kRowList;  // the same in every wave
   if (ok) {
+    // Fewer listed tokens than k: no segment had k finite logits, so every finite one is listed,
+    // and the cutoff at their number keeps them all, as the row's own does.
+    k = min(k, total);
     constexpr int kOwn = kRowList / kThreads;
     const uint2* lists = p.list + row * n * int64_t(kSegList);
     uint2 own[kOwn];
@@ -1446,10 +1460,10 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
         const float inv_z = 1.f / z;
         const bool done =
             kept <= kWave
-                ? finish_wave<1>(a, row, cand_i, cand_s, kept, m, inv_z, r.top_k, r.top_p, listed_to)
+                ? finish_wave<1>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p, listed_to)
             : kept <= 2 * kWave
-                ? finish_wave<2>(a, row, cand_i, cand_s, kept, m, inv_z, r.top_k, r.top_p, listed_to)
-                : finish_wave<4>(a, row, cand_i, cand_s, kept, m, inv_z, r.top_k, r.top_p,
+                ? finish_wave<2>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p, listed_to)
+                : finish_wave<4>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p,
                                  listed_to);
         if (lane == 0) sh.ok = done;
       }
@@ -1458,7 +1472,7 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     } else {
       // The whole workgroup, where the bound itself shows the lists complete.
       ok = kept <= kCandidates && listed_to <= edge &&
-           finish_candidates(sh.row, a, row, cand_i, cand_s, cand_p, kept, m, 1.f / z, r.top_k,
+           finish_candidates(sh.row, a, row, cand_i, cand_s, cand_p, kept, m, 1.f / z, k,
                              r.top_p);
     }
   }

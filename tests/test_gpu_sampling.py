@@ -291,3 +291,29 @@ def test_split_workspace_is_checked(gpu):
     assert b"workspace" in lib().mi355x_sample_split(*args, ws.data_ptr(), need - 1, stream)
     assert b"workspace" in lib().mi355x_sample_split(*args, None, need, stream)
     assert lib().mi355x_sample_split(*args, ws.data_ptr(), need, stream) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("allowed", [1, 4, 30, 49, 50, 51, 127, 128, 300])
+@pytest.mark.parametrize("spread", [1.0, 10.0, 40.0])
+def test_split_rows_with_few_or_negligible_tokens(gpu, dtype, allowed, spread):
+    """Fewer finite logits than k, as many and a few more, spread over the row or side by side,
+    with a k-th probability that does or does not reach the fixed-point mass; masks of -inf and of
+    the type's lowest value. Equal ids with one workgroup per row."""
+    rows, vocab = 2 * len(ROW_KINDS), 40000
+    g = torch.Generator().manual_seed(allowed + int(spread))
+    values = torch.randn(rows, vocab, generator=g) * spread
+    mask = torch.ones(rows, vocab, dtype=torch.bool)
+    for r in range(rows):
+        if r % 2:
+            mask[r, 777 * r:777 * r + allowed] = False
+        else:
+            mask[r, torch.randperm(vocab, generator=g)[:allowed]] = False
+    params = [ROW_KINDS[i % len(ROW_KINDS)] for i in range(rows)]
+    for hidden in (float("-inf"), torch.finfo(dtype).min):
+        logits = values.to(dtype).masked_fill(mask, hidden).to(gpu)
+        got = Sampler(allowed).sample_batch_device(logits, params)
+        assert torch.equal(got, one_workgroup_per_row(logits, params, allowed, 0))
+    logits = values.to(dtype).to(gpu)
+    got = Sampler(allowed).sample_batch_device(logits, params)
+    assert torch.equal(got, one_workgroup_per_row(logits, params, allowed, 0))
