@@ -65,9 +65,15 @@ static_assert(kDmaMaxEntries % 64 == 0, "entries are staged 64 at a time");
 // 29.4 -> 27.1, 16 MB 16.0 -> 15.0; 5.5 MB, still found in the cache, 12.4 -> 12.8.
 constexpr int64_t kOnceBytes = int64_t(8) << 20;
 constexpr float kLog2e = 1.4426950408889634f;
-// Up to this batch a merge workgroup serves one head: the grid has at least 256 workgroups
-// either way above it, and a request is cut into at most 8 chunks or so, one round of loads.
+// Up to this batch the merge gives every (request, q head) four waves. Above it that grid costs a
+// plan with few chunks per request more than it gives (256 requests of about 100 tokens at Hq 32,
+// store + decode + merge: 31.6 us against 30.5 with one wave each), so only the requests of more
+// than kLongChunks chunks, kLongSlots at most, get four.
 constexpr int64_t kWideMergeRows = 32;
+constexpr int kLongChunks = 16;
+constexpr int kLongSlots = 16;
+constexpr int kHeaderInts = 24;
+static_assert(kHeaderInts >= 5 + kLongSlots && kHeaderInts % 4 == 0, "the header's lists");
 
 // ---------------------------------------------------------------------------
 // Device buffer with geometric growth, matching the reference workspace rule
@@ -115,7 +121,9 @@ struct DeviceBuffer {
 //   [0]                  number of workgroups (per kv-head slice)
 //   [1]                  number of work items
 //   [2]                  1: the K/V copies are non-temporal (kOnceBytes)
-//   [4, 4+B+1)           indptr
+//   [3]                  most chunks of a request whose heads take one merge wave each
+//   [4]                  number of requests with more, and [5, 5+kLongSlots) those requests
+//   [kHeaderInts, +B+1)  indptr
 //   [o_work, +4*cap)     work items {request, token_begin, token_end, partial}
 //   [o_merge, +2*B)      per-request {first partial, chunk count}
 //   [o_wg, +wgs+1)       first work item of each workgroup
@@ -130,7 +138,7 @@ struct IntLayout {
   int64_t o_indptr, o_work, o_merge, o_wg, o_wgrec, total;
   static IntLayout make(int64_t rows, int64_t items_cap, int64_t wg_cap) {
     IntLayout l{};
-    l.o_indptr = 4;
+    l.o_indptr = kHeaderInts;
     l.o_work = (l.o_indptr + rows + 1 + 3) / 4 * 4;
     l.o_merge = l.o_work + 4 * items_cap;
     l.o_wg = l.o_merge + 2 * rows;
@@ -149,7 +157,7 @@ struct DecodePlan {
   int64_t graph_rows = 0, graph_columns = 0;
   // Current plan facts.
   int64_t batch = 0, total_pages = 0, num_items = 0, chunk_tokens = 0, items_capacity = 0;
-  int64_t num_wgs = 0, wg_capacity = 0;
+  int64_t num_wgs = 0, wg_capacity = 0, num_long = 0;
   int64_t cus = 0;
   IntLayout layout{};
   DeviceBuffer ints, indices, last_len, partial_o, partial_lse;
@@ -252,7 +260,8 @@ LaunchShape launch_shape(int64_t cus, int64_t num_kv_heads, int64_t page_size) {
     s.max_item = std::numeric_limits<int32_t>::max();
     s.tile = kTileTokens;
   }
-  // Every workgroup but the last takes more than share - 32 >= 3/4 share tokens.
+  // schedule() takes the smallest share whose walk needs at most `workgroups` workgroups; the room
+  // above them is for the walks it tries, which stop there.
   s.wg_capacity = s.workgroups + s.workgroups / 3 + 2;
   return s;
 }
@@ -1178,18 +1187,15 @@ __global__ __launch_bounds__(64 * W, 1) void decode_mma_kernel(DecodeArgs a) {
 
 // Split-KV merge, two dims per lane: chunks are combined with a running log2-sum-exp, the
 // loads of kUnroll chunks in flight together. Bound by the latency of its rounds of loads.
-// WAVES = 1: one wave per (request, q head), four heads per workgroup. WAVES = 4: a workgroup
-// per (request, q head), wave w taking every fourth group of kUnroll chunks, joined through
-// LDS: batches of few requests are cut into up to a few hundred chunks each (one request of
-// 32,768 tokens, 256 chunks, store + decode + merge: 44.5 us against 60.6 with one wave).
+// WAVES = 1: one wave for one q head of a request; WAVES = 4: wave w takes every fourth group of
+// kUnroll chunks, joined through LDS. Requests alone in their batch are cut into up to a few
+// hundred chunks (one request of 32,768 tokens, 256 chunks, store + decode + merge: 44.5 us with
+// four waves against 60.6 with one).
 template <int DT, int WAVES>
-__global__ __launch_bounds__(256) void merge_kernel(DecodeArgs a, int32_t rows) {
+__device__ __forceinline__ void merge_head(const DecodeArgs& a, int req, int qh) {
   static_assert(WAVES == 1 || WAVES == 4, "a workgroup holds four waves");
   const int wave = threadIdx.x >> 6;
-  const int req = blockIdx.x;
-  const int qh = WAVES == 1 ? blockIdx.y * 4 + wave : blockIdx.y;
   const int lane = threadIdx.x & 63;
-  if (req >= rows || qh >= a.num_q_heads) return;
   const int first = a.ints[a.o_merge + 2 * req];
   const int count = a.ints[a.o_merge + 2 * req + 1];
   if (count <= 1) return;
@@ -1249,15 +1255,44 @@ __global__ __launch_bounds__(256) void merge_kernel(DecodeArgs a, int32_t rows) 
       packed;
 }
 
+// Few requests: a workgroup per (request, q head).
 template <int DT>
-void launch_merge(const DecodeArgs& a, int64_t batch, int64_t num_q_heads, hipStream_t s) {
-  const auto rows = static_cast<uint32_t>(batch);
-  const auto heads = static_cast<uint32_t>(num_q_heads);
+__global__ __launch_bounds__(256) void merge_wide_kernel(DecodeArgs a) {
+  merge_head<DT, 4>(a, blockIdx.x, blockIdx.y);
+}
+
+// Many: the first long_slots * Hq workgroups take a head each of the requests listed as long, the
+// others four heads of any other request. us, store + decode + merge at Hq 32 on a graph plan,
+// one wave per head throughout -> this: 8,192 tokens beside 32 requests of 16 30.7 -> 19.4, 32,768
+// beside 39 of 64 52.2 -> 38.0, 4 of 4,096 beside 200 of 200 52.8 -> 52.3, and with none long 100
+// requests of 100 to 2,971 105.0 -> 105.4, 256 of about 100 30.4 -> 30.7.
+template <int DT>
+__global__ __launch_bounds__(256) void merge_kernel(DecodeArgs a, int32_t long_slots) {
+  const int long_wgs = long_slots * a.num_q_heads;
+  const int wg = blockIdx.x;
+  if (wg < long_wgs) {
+    const int slot = wg / a.num_q_heads;
+    if (slot < a.ints[4]) merge_head<DT, 4>(a, a.ints[5 + slot], wg - slot * a.num_q_heads);
+    return;
+  }
+  const int groups = (a.num_q_heads + 3) / 4;
+  const int req = (wg - long_wgs) / groups;
+  const int qh = ((wg - long_wgs) - req * groups) * 4 + (threadIdx.x >> 6);
+  if (qh >= a.num_q_heads || a.ints[a.o_merge + 2 * req + 1] > a.ints[3]) return;
+  merge_head<DT, 1>(a, req, qh);
+}
+
+// long_slots: what the grid holds for long requests. A graph plan's launch is fixed when it is
+// captured, so its grid holds kLongSlots.
+template <int DT>
+void launch_merge(const DecodeArgs& a, int64_t batch, int64_t long_slots, hipStream_t s) {
+  const int64_t heads = a.num_q_heads;
   if (batch <= kWideMergeRows)
-    merge_kernel<DT, 4><<<dim3(rows, heads), dim3(256), 0, s>>>(a, static_cast<int32_t>(batch));
+    merge_wide_kernel<DT><<<dim3(static_cast<uint32_t>(batch), static_cast<uint32_t>(heads)),
+                            dim3(256), 0, s>>>(a);
   else
-    merge_kernel<DT, 1><<<dim3(rows, (heads + 3) / 4), dim3(256), 0, s>>>(
-        a, static_cast<int32_t>(batch));
+    merge_kernel<DT><<<dim3(static_cast<uint32_t>(long_slots * heads + batch * ((heads + 3) / 4))),
+                       dim3(256), 0, s>>>(a, static_cast<int32_t>(long_slots));
 }
 
 // Tokens per 16-lane group per loop trip. Override with MI355X_DECODE_U
@@ -1509,6 +1544,22 @@ extern "C" void* mi355x_decode_prepare(void* existing, const int32_t* block_tabl
     int64_t tokens = 0;
     for (int64_t r = 0; r < batch; ++r) tokens += plan->host_lengths[r];
     host[2] = tokens * num_kv_heads * kHeadDim * 4 >= kOnceBytes;
+    // Requests that the merge gives four waves a head: those of more than kLongChunks chunks, or
+    // of twice as many as often as it takes to fit the list (a batch of very long requests).
+    const int32_t* merge = host + layout.o_merge;
+    host[3] = kLongChunks;
+    int64_t longs = 0;
+    for (int64_t r = 0; r < batch; ++r) {
+      if (merge[2 * r + 1] <= host[3]) continue;
+      if (longs < kLongSlots) {
+        host[5 + longs++] = static_cast<int32_t>(r);
+      } else {
+        host[3] *= 2;
+        longs = 0;
+        r = -1;
+      }
+    }
+    host[4] = static_cast<int32_t>(longs);
     // Start records: the first item of each workgroup and the page-entry index of its
     // first token (pack_page_metadata fills the slots from the block table).
     for (int64_t w = 0; w < wgs; ++w) {
@@ -1553,6 +1604,7 @@ extern "C" void* mi355x_decode_prepare(void* existing, const int32_t* block_tabl
     plan->chunk_tokens = chunk;
     plan->items_capacity = items_cap;
     plan->num_wgs = wgs;
+    plan->num_long = longs;
     plan->wg_capacity = wg_cap;
     plan->layout = layout;
     created.release();
@@ -1662,10 +1714,11 @@ extern "C" const char* mi355x_decode_run(const void* plan_ptr, const void* q, in
   if (!ok) return set_error("unsupported query group size");
   if (const char* err = launch_status("decode_kernel")) return err;
   if (p.graph || p.num_items > p.batch) {  // some request was split
+    const int64_t long_slots = p.graph ? kLongSlots : p.num_long;
     if (dtype == 0)
-      launch_merge<0>(a, batch, num_q_heads, s);
+      launch_merge<0>(a, batch, long_slots, s);
     else
-      launch_merge<1>(a, batch, num_q_heads, s);
+      launch_merge<1>(a, batch, long_slots, s);
     return launch_status("merge_kernel");
   }
   return nullptr;

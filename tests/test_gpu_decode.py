@@ -301,7 +301,7 @@ def test_small_batches_spread_thin(gpu, hq, hkv, rows, lo, hi):
 
 def test_graph_plan_crosses_the_non_temporal_size(gpu):
     """One graph plan re-planned at lengths whose K/V is below, just at and above 8 MiB (2,048
-    tokens of 8 kv heads): the copies' hint travels with the plan, the results do not change."""
+    tokens of 8 kv heads): the results do not depend on which copies a replay takes."""
     g = torch.Generator().manual_seed(8)
     rng = np.random.default_rng(8)
     _, table, kc, vc, q = _random_decode_case(gpu, g, rng, 2, 32, 8, 16, 1600, 1600, 300,
@@ -320,3 +320,60 @@ def test_graph_plan_crosses_the_non_temporal_size(gpu):
         out = batch.forward(q, q, q, cache)
         want = oatt.decode_with_cache(f32(q), f32(kc), f32(vc), table, lens, 16)
         assert_close(f32(out).reshape(want.shape), want, f"lens {lens}")
+
+
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (16, 8), (6, 6)])
+def test_long_requests_among_many_short_ones(gpu, hq, hkv):
+    """More than 32 requests, some cut into far more chunks than the others (at the front, in the
+    middle and at the end, none, two, all alike), eager and on one graph plan re-planned for each:
+    every head of every request is merged once."""
+    rows, most = 33, 8192
+    g = torch.Generator().manual_seed(hq)
+    rng = np.random.default_rng(hq)
+    _, table, kc, vc, q = _random_decode_case(gpu, g, rng, rows, hq, hkv, 16, most, most,
+                                              600, torch.bfloat16)
+    attn = make_backend(gpu, hq, hkv, 16)
+    cache = BaseAttention()
+    cache.bind_kv_cache(kc, vc)
+    lengths = torch.ones(rows, dtype=torch.int32, device=gpu)
+    meta = AttentionMetadata(BatchPhase.DECODE, block_table=torch.from_numpy(table).to(gpu),
+                             cache_seqlens=lengths)
+    state = attn.prepare_decode_graph(meta)
+    graph = attn.prepare(meta, rows)
+    out = torch.empty(rows, hq * 128, dtype=torch.bfloat16, device=gpu)
+    for long in ({7: 8192}, {0: 5000, 32: 4099}, {}, {32: 8191}, dict.fromkeys(range(33), 900)):
+        lens = np.array([long.get(r, 1 + r % 17) for r in range(rows)], dtype=np.int32)
+        lengths.copy_(torch.from_numpy(lens))
+        state.prepare_replay(DecodeHostMetadata(lens.tolist()))
+        eager = make_backend(gpu, hq, hkv, 16).prepare(
+            AttentionMetadata(BatchPhase.DECODE, block_table=meta.block_table,
+                              cache_seqlens=lengths), rows)
+        want = oatt.decode_with_cache(f32(q), f32(kc), f32(vc), table, lens, 16)
+        for batch in (graph, eager):
+            batch.forward_into(q, q, q, cache, out.fill_(float("nan")))
+            assert_close(f32(out).reshape(want.shape), want, f"long {long}")
+
+
+def test_more_long_requests_than_the_merge_lists(gpu):
+    """33 requests of up to 35,000 single-token pages, an item holding 2,047 of them: all are cut
+    into more chunks than a merge wave takes, more of them than the plan lists."""
+    rows, most, heads = 33, 35000, 4
+    g = torch.Generator().manual_seed(33)
+    kc, vc = (randn((most + 1, 1, heads, 128), g, torch.bfloat16, gpu) for _ in range(2))
+    q = randn((rows, heads, 128), g, torch.bfloat16, gpu)
+    row = torch.randperm(most, generator=g).to(torch.int32).to(gpu) + 1
+    lens = [most - 97 * r for r in range(rows)]
+    cache = BaseAttention()
+    cache.bind_kv_cache(kc, vc)
+    batch = make_backend(gpu, heads, heads, 1).prepare(
+        AttentionMetadata(BatchPhase.DECODE, block_table=row.repeat(rows, 1),
+                          cache_seqlens=torch.tensor(lens, dtype=torch.int32, device=gpu)), rows)
+    counts = np.asarray(batch.plan.plan.read_metadata()["merge"]).reshape(rows, 2)[:, 1]
+    assert (counts > 16).sum() > 16
+    out = torch.full((rows, heads * 128), float("nan"), dtype=torch.bfloat16, device=gpu)
+    batch.forward_into(q, q, q, cache, out)
+    k, v = kc[row.long(), 0].float(), vc[row.long(), 0].float()
+    for r, n in enumerate(lens):
+        p = torch.softmax((k[:n] * q[r].float()).sum(-1) * 128 ** -0.5, 0)
+        want = (p.unsqueeze(-1) * v[:n]).sum(0)
+        assert_close(f32(out[r]), f32(want), f"request {r} of {n}")
