@@ -116,22 +116,25 @@ class Sampler:
                 and len(objs) == len(params_list)
                 and all(a is b for a, b in zip(params_list, objs))):
             return self._params
-        normalized = [p.normalized() for p in params_list]
-        key = (device, tuple((p.temperature, p.top_k, p.top_p) for p in normalized))
+        # Plain walks over the fields (``normalized`` would copy every object): a batch whose
+        # members changed comes here on each step that a request joins or leaves.
+        temps = [p.temperature for p in params_list]
+        ks = [p.top_k for p in params_list]
+        ps = [p.top_p if 0.0 <= p.top_p <= 1.0 else 1.0 for p in params_list]
+        key = (device, temps, ks, ps)
         if key != self._param_key:
-            n = len(normalized)
+            n = len(temps)
             host = torch.empty(3 * n, dtype=torch.float32, pin_memory=True)
-            host[:n] = torch.tensor([p.temperature for p in normalized], dtype=torch.float32)
-            host[2 * n:] = torch.tensor([p.top_p for p in normalized], dtype=torch.float32)
-            ks = torch.tensor([p.top_k for p in normalized], dtype=torch.int32)
-            host[n:2 * n] = ks.view(torch.float32)  # bit-copy the int32 top-k
+            k = torch.tensor(ks, dtype=torch.int32)
+            torch.cat((torch.tensor(temps, dtype=torch.float32), k.view(torch.float32),
+                       torch.tensor(ps, dtype=torch.float32)), out=host)  # top-k bit for bit
             dev = host.to(device, non_blocking=True)
             self._params = (dev[:n], dev[n:2 * n].view(torch.int32), dev[2 * n:])
-            drawn = [p for p in normalized if p.temperature > 0 and p.top_p > 0]
-            self._top_p_rows = any(p.top_p < 1 and (p.top_k <= 0 or p.top_k > LISTED_TOP_K)
-                                   for p in drawn)
+            drawn = [(k, p) for t, k, p in set(zip(temps, ks, ps)) if t > 0 and p > 0]
+            large = [k for k, _ in drawn if k > LISTED_TOP_K]
+            self._top_p_rows = any(p < 1 and (k <= 0 or k > LISTED_TOP_K) for k, p in drawn)
             self._all_greedy = not drawn
-            self._large_k = min((p.top_k for p in drawn if p.top_k > LISTED_TOP_K), default=None)
+            self._large_k = min(large, default=None)
             self._param_key = key
         self._param_objs = tuple(params_list)  # last: a build that raised is not taken for built
         return self._params
