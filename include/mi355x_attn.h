@@ -352,12 +352,14 @@ const char* mi355x_sample(const void* logits, int64_t rows, int64_t vocab, int64
                           void* stream);
 
 /* mi355x_sample with each row spread over several workgroups (a few rows leave most of the
- * chip idle otherwise, and a row is read once instead of two to five times): the same rules,
- * cutoffs and draws. Partial results go to `workspace` (16-byte aligned,
- * mi355x_sample_workspace_bytes of the same rows, vocab and top_p_rows; contents undefined
- * before and after; calls that overlap need workspaces of their own). top_p_rows says that
- * some row may be cut by top_p with no top_k below vocab: such rows take three more launches
- * and, when it is false, one workgroup each, with the same result. */
+ * chip idle otherwise): the same rules and draws, and the same cutoffs up to the fp32 rounding
+ * of the sum of exponentials, which is joined from the workgroups' sums. A row is read once,
+ * or, where it is cut by top_p with no top_k below vocab, four times (five for fp32). Partial
+ * results go to `workspace` (16-byte aligned, mi355x_sample_workspace_bytes of the same rows,
+ * vocab and top_p_rows; contents undefined before and after; calls that overlap need workspaces
+ * of their own). top_p_rows says that some row may be cut by top_p with no top_k below vocab:
+ * such rows take three more launches (four for fp32) and, when it is false, one workgroup each,
+ * with the result of mi355x_sample. */
 const char* mi355x_sample_split(const void* logits, int64_t rows, int64_t vocab,
                                 int64_t row_stride, int dtype, const float* temperature,
                                 const int32_t* top_k, const float* top_p, uint64_t seed,
@@ -365,7 +367,10 @@ const char* mi355x_sample_split(const void* logits, int64_t rows, int64_t vocab,
                                 int64_t workspace_bytes, void* stream);
 
 /* Workspace bytes of mi355x_sample_split; 0 when it does not take the shape (more than 1,024
- * rows, up to 16,384 columns or more than 2.1 million): use mi355x_sample. Host-only. */
+ * rows, up to 16,384 columns or more than 2.1 million): use mi355x_sample. About 4 KiB per
+ * workgroup, which takes up to 8,192 logits, and with top_p_rows 48 KiB per row: for rows of
+ * 151,936 logits 1.8 MB at 5 rows, 33 MB at 256, 132 MB at 1,024; 1.15 GB at most (1,024 rows
+ * of 2 million). Host-only. */
 int64_t mi355x_sample_workspace_bytes(int64_t rows, int64_t vocab, bool top_p_rows);
 
 #pragma GCC visibility pop

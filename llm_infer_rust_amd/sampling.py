@@ -11,10 +11,11 @@ Mirrors ``src/engine/sampling.rs``:
   step's embedding, ``finish()`` waits and validates.
 
 Unlike the reference, which groups rows by identical parameters and launches
-one FlashInfer call per group (``:343-371``), one kernel launch serves the
+one FlashInfer call per group (``:343-371``), one library call serves the
 whole heterogeneous batch: the parameters travel as per-row device arrays.
-The random stream is (seed, offset): ``manual_seed`` resets both and every
-sampling launch advances the offset by one.
+The call is one launch, or two to six where rows are spread over several
+workgroups. The random stream is (seed, offset): ``manual_seed`` resets both
+and every sampling call advances the offset by one.
 """
 from __future__ import annotations
 
@@ -92,7 +93,7 @@ class PendingSample:
 
 
 class Sampler:
-    """Samples one next-token id per logits row, whole batch in one launch."""
+    """Samples one next-token id per logits row, the whole heterogeneous batch in one call."""
 
     def __init__(self, seed: int = 0):
         self.manual_seed(seed)
@@ -159,8 +160,13 @@ class Sampler:
         if ((self._large_k is None or self._large_k >= logits.size(1))
                 and not (self._all_greedy and rows >= GREEDY_ROWS)):
             need = lib().mi355x_sample_workspace_bytes(rows, logits.size(1), self._top_p_rows)
+        ws = None
         if need:
-            ws = torch.empty(need, dtype=torch.uint8, device=logits.device)
+            try:
+                ws = torch.empty(need, dtype=torch.uint8, device=logits.device)
+            except torch.OutOfMemoryError:
+                pass  # one workgroup per row needs no workspace
+        if ws is not None:
             check(lib().mi355x_sample_split(*args, self._top_p_rows, ws.data_ptr(), need,
                                             stream_of(logits)), "sample")
         else:

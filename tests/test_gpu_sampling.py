@@ -317,3 +317,23 @@ def test_split_rows_with_few_or_negligible_tokens(gpu, dtype, allowed, spread):
     logits = values.to(dtype).to(gpu)
     got = Sampler(allowed).sample_batch_device(logits, params)
     assert torch.equal(got, one_workgroup_per_row(logits, params, allowed, 0))
+
+
+def test_sampling_without_room_for_the_split_workspace(gpu, monkeypatch):
+    """A batch that was sampled before rows were split is still sampled when there is no memory
+    left for the split call's workspace."""
+    g = torch.Generator().manual_seed(40)
+    logits = torch.randn(len(ROW_KINDS), 40000, generator=g).to(torch.bfloat16).to(gpu)
+    real = torch.empty
+
+    def full(*args, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return real(*args, **kw)
+
+    s = Sampler(3)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", full)
+        got = s.sample_batch_device(logits, ROW_KINDS)
+    assert s.offset == 1
+    assert torch.equal(got, one_workgroup_per_row(logits, ROW_KINDS, 3, 0))
