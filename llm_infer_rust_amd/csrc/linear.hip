@@ -29,6 +29,7 @@
 #include <cmath>
 #include <mutex>
 #include <cstdint>
+#include <type_traits>
 
 #include "common.h"
 
@@ -158,11 +159,13 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void linear_kernel(LinearArgs a) {
     kt = a.tiles_m == 1 || a.K > 4096 ? phase % n_k : (phase & 7) * n_k / 8;
   }
   // Weights that are read once are copied non-temporally and leave L2 to x (gate_up at 24 rows
-  // 38.8 -> 35.3 us); keep_weights is the host's word that several M tiles read them from L2.
-  auto issue = [&](int stage) {
+  // 38.8 -> 35.3 us); keep_weights is the host's word that several M tiles read them from L2. It
+  // is asked once, outside the K loop (gate_up 6144 x 1024 at one row 7.9 us with the question at
+  // every copy, 7.4 so).
+  auto issue = [&](int stage, auto keep) {
 #pragma unroll
     for (int j = 0; j < kCopies; ++j) {
-      if (8 * (wave + NW * j) < BM || a.keep_weights)
+      if (decltype(keep)::value || 8 * (wave + NW * j) < BM)
         copy_to_lds(src[j] + kt * kBK, dst[j] + stage * kStageBytes);
       else
         copy_to_lds_nt(src[j] + kt * kBK, dst[j] + stage * kStageBytes);
@@ -210,18 +213,24 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void linear_kernel(LinearArgs a) {
         for (int j = 0; j < B_BLK; ++j) acc[i][j] = mfma32<DT>(af[kk][i], bf[kk][j], acc[i][j]);
   };
 
+  auto stream = [&](auto keep) {
 #pragma unroll
   for (int st = 0; st < STAGES - 1; ++st)
-    if (st < n_k) issue(st);
+    if (st < n_k) issue(st, keep);
   int read_stage = 0, fill_stage = STAGES - 1;
   for (int t = 0; t < n_k; ++t) {
     wait_tiles_ahead<kCopies, STAGES - 2>(min(STAGES - 2, n_k - 1 - t));
     __syncthreads();
-    if (t + STAGES - 1 < n_k) issue(fill_stage);
+    if (t + STAGES - 1 < n_k) issue(fill_stage, keep);
     compute(read_stage);
     read_stage = read_stage == STAGES - 1 ? 0 : read_stage + 1;
     fill_stage = fill_stage == STAGES - 1 ? 0 : fill_stage + 1;
   }
+  };
+  if (a.keep_weights)
+    stream(std::true_type{});
+  else
+    stream(std::false_type{});
 
   // Lane holds D[n][m] for m = column `col` of each B block and n = 8 q + 4 half + e
   // (e = 0..3) of each A block, accumulator elements 4 q + e.
