@@ -231,7 +231,7 @@ bool head_views_vectorisable(const HeadArgs& a) {
 // SiLU(gate) * up with one 128-bit chunk of gate, up and out per thread. Bound by HBM. ID is the
 // index type: the division by the row's chunks is done in 32 bits where the chunks can be
 // counted in them (in 64 bits it alone held the pass at 5.0 TB/s: 8,192 rows of 12,288 columns,
-// 119.6 -> 102.8 us). ONCE marks a launch whose tensors outgrow the Infinity Cache (kOnceBytes):
+// 119.6 -> 102.8 us). ONCE marks a launch whose gate_up outgrows the Infinity Cache (kOnceBytes):
 // gate_up is read with non-temporal loads (102.8 -> 99.5 us). The stores stay plain: without a
 // place in the cache the pass itself is quicker (94.3 us), and the product that reads out next
 // loses more (gate_up GEMM + pass + down GEMM 1,723 us with neither hint, 1,705 with the loads,
@@ -254,9 +254,9 @@ __global__ __launch_bounds__(256) void silu_mul_vec(const uint16_t* __restrict__
   st128(out + static_cast<int64_t>(id) * 8, pack8<DT>(y));
 }
 
-// From this many bytes of gate_up and out they outgrow the 256 MiB Infinity Cache, and gate_up's
-// place in it is worth more to out. Below it the loads find gate_up there and the hint costs
-// (512 rows: 7.7 us against 8.7).
+// From this many bytes of gate_up it outgrows the 256 MiB Infinity Cache, and its place in it is
+// worth more to out. Below it the loads find gate_up there and the hint costs (512 rows of 12,288
+// 7.7 us against 8.7, 16,384 of 3,072, 192 MiB, 48.8 against 53.4).
 constexpr int64_t kOnceBytes = int64_t(256) << 20;
 
 template <int DT>
@@ -266,7 +266,7 @@ void launch_silu_vec(const uint16_t* in, uint16_t* out, int64_t tokens, int64_t 
   const dim3 grid(static_cast<uint32_t>((total + 255) / 256));
   if (total > INT32_MAX)
     silu_mul_vec<DT, int64_t, true><<<grid, dim3(256), 0, s>>>(in, out, total, width);
-  else if (total * 48 >= kOnceBytes)
+  else if (total * 32 >= kOnceBytes)
     silu_mul_vec<DT, uint32_t, true>
         <<<grid, dim3(256), 0, s>>>(in, out, static_cast<uint32_t>(total), width);
   else
