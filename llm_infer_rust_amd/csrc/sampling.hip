@@ -236,8 +236,7 @@ __device__ __forceinline__ float candidate_edge(float s_k, float m) {
 
 // Both cutoffs and the draw among n gathered candidates (cand_p is scratch; the lists are in
 // LDS and complete: every token of the row whose p can reach the k-th largest is listed).
-// False, and nothing written, when fewer than k candidates exist or the k-th p has no
-// fixed-point mass under a top-p cutoff. All kThreads threads call it.
+// False, and nothing written, when fewer than k candidates exist. All kThreads threads call it.
 __device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& a, int64_t row,
                                                   const uint32_t* cand_i, const float* cand_s,
                                                   float* cand_p, uint32_t n, float m, float inv_z,
@@ -263,7 +262,7 @@ __device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& 
   }
   __syncthreads();
   const float p_k = sh.red_f[0];
-  if (!sh.k_found || (use_p && fixed_mass(p_k) == 0)) return false;
+  if (!sh.k_found) return false;
   float cut = p_k;
   if (use_p) {
     // Mass at or above p_k; when it reaches top_p, the top-p cutoff is the largest
@@ -289,6 +288,15 @@ __device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& 
       int64_t bi = 0;
       block_argmax(sh, bv, bi);
       cut = bv;
+    } else if (fixed_mass(p_k) == 0) {
+      // Rounding kept the whole mass below the target, and all of it lies above p_k: the cutoff
+      // is the lowest p that has any.
+      float low = -INFINITY;
+      for (uint32_t t = threadIdx.x; t < n; t += kThreads)
+        if (fixed_mass(cand_p[t])) low = fmaxf(low, -cand_p[t]);
+      int64_t bi = 0;
+      block_argmax(sh, low, bi);
+      cut = -low;
     }
   }
   // The race over the surviving candidates (order-independent: larger key, then lower index).
@@ -638,7 +646,7 @@ constexpr int kMaxChunks = 4;             // steps held in registers (8: half th
 constexpr int kMaxSegments = 256;         // per row
 constexpr uint32_t kSegList = 512;        // listed tokens per segment
 constexpr int64_t kSplitTopK = 128;       // largest k of the segment lists
-constexpr uint32_t kRowList = 8192;       // listed tokens per row
+constexpr uint32_t kRowOwn = 8192;        // listed tokens of a row loaded before the bound is known
 constexpr int kSegPeaks = kSegThreads / 16;
 constexpr int kLevelBins = 1024;          // bins of the levels after the first
 
@@ -1218,91 +1226,55 @@ __global__ __launch_bounds__(kSegThreads) void race_segments(SampleArgs a, Split
   }
 }
 
-// finish_candidates for at most 64 R candidates by one wave, each pair compared through lane
+// finish_candidates for at most kWave candidates by one wave, each pair compared through lane
 // broadcasts: with 60 candidates 4 us against the workgroup-wide version's 16 (its LDS round
-// trips). False as well when tokens that could share the k-th p may not have been listed, the
-// lists being complete down to listed_to only.
-template <int R>
+// trips), which is the quicker one from 64 (top-k 100 of 16,385: 36.8 us a call with two to four
+// candidates a lane, 23.4 workgroup-wide). False as well when tokens that could share the k-th p
+// may not have been listed, the lists being complete down to listed_to only.
 __device__ bool finish_wave(const SampleArgs& a, int64_t row, const uint32_t* cand_i,
                             const float* cand_s, uint32_t n, float m, float inv_z, int64_t top_k,
                             float top_p, float listed_to) {
-  const int lane = threadIdx.x % kWave;
+  const uint32_t lane = threadIdx.x % kWave;
   const bool use_p = top_p < 1.f;
   const uint32_t k = static_cast<uint32_t>(top_k);
-  float s[R], p[R];
-  uint32_t gt[R], ge[R];
-  unsigned long long fx[R], mass[R];  // mass at or above the own p
-#pragma unroll
-  for (int t = 0; t < R; ++t) {
-    const uint32_t c = lane + kWave * t;
-    s[t] = c < n ? cand_s[c] : -INFINITY;
-    p[t] = c < n ? probability(s[t], m, inv_z) : -1.f;
-    fx[t] = c < n ? fixed_mass(p[t]) : 0ull;
-    gt[t] = ge[t] = 0;
-    mass[t] = 0;
+  const float s = lane < n ? cand_s[lane] : -INFINITY;
+  const float p = lane < n ? probability(s, m, inv_z) : -1.f;
+  const unsigned long long fx = lane < n ? fixed_mass(p) : 0ull;
+  uint32_t gt = 0, ge = 0;
+  unsigned long long mass = 0;  // at or above the own p
+  for (uint32_t u = 0; u < n; ++u) {
+    const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), u));
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx), u);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx >> 32), u);
+    const unsigned long long f = (static_cast<unsigned long long>(hi) << 32) | lo;
+    gt += v > p;
+    ge += v >= p;
+    mass += v >= p ? f : 0ull;
   }
-#pragma unroll
-  for (int t = 0; t < R; ++t) {
-    const int some = min(kWave, static_cast<int>(n) - kWave * t);
-    for (int u = 0; u < some; ++u) {
-      const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p[t]), u));
-      const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx[t]), u);
-      const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx[t] >> 32), u);
-      const unsigned long long f = (static_cast<unsigned long long>(hi) << 32) | lo;
-#pragma unroll
-      for (int w = 0; w < R; ++w) {
-        gt[w] += v > p[w];
-        const bool above = v >= p[w];
-        ge[w] += above;
-        mass[w] += above ? f : 0ull;
-      }
-    }
-  }
-  // The k-th largest p and the mass at or above it.
-  float p_k = -1.f;
-  bool reached = false;
-#pragma unroll
-  for (int t = 0; t < R; ++t)
-    if (p[t] >= 0.f && gt[t] < k && ge[t] >= k) {
-      p_k = p[t];
-      reached = mass[t] >= mass_target(top_p);
-    }
-  reached = __any(reached);
-  p_k = wave_max(p_k);
+  // The k-th largest p, the mass at or above it, and the lowest s that has it.
+  const bool is_k = p >= 0.f && gt < k && ge >= k;
+  const float p_k = wave_max(is_k ? p : -1.f);
+  const bool reached = __any(is_k && mass >= mass_target(top_p));
   if (p_k < 0.f) return false;
-  float s_k = INFINITY;  // the lowest s that has it
-#pragma unroll
-  for (int t = 0; t < R; ++t)
-    if (p[t] == p_k) s_k = fminf(s_k, s[t]);
-  s_k = -wave_max(-s_k);
+  const float s_k = -wave_max(p == p_k ? -s : -INFINITY);
   if (listed_to > candidate_edge(s_k, m)) return false;
   float cut = p_k;
-  if (use_p && reached) {
-#pragma unroll
-    for (int t = 0; t < R; ++t)
-      if (p[t] > cut && mass[t] >= mass_target(top_p)) cut = p[t];
-    cut = wave_max(cut);
-  } else if (use_p && fixed_mass(p_k) == 0) {
+  if (use_p && reached)
+    cut = wave_max(p > cut && mass >= mass_target(top_p) ? p : cut);
+  else if (use_p && fixed_mass(p_k) == 0)
     // Rounding kept the whole mass below the target, and all of it lies above p_k: the cutoff is
     // the lowest p that has any.
-    float low = INFINITY;
-#pragma unroll
-    for (int t = 0; t < R; ++t)
-      if (fx[t]) low = fminf(low, p[t]);
-    cut = -wave_max(-low);
-  }
+    cut = -wave_max(fx ? -p : -INFINITY);
   float best = -INFINITY;
   uint32_t best_i = static_cast<uint32_t>(a.vocab);
-#pragma unroll
-  for (int t = 0; t < R; ++t) {
-    if (!(p[t] > 0.f && p[t] >= cut)) continue;
-    const uint32_t i = cand_i[lane + kWave * t];
+  if (p > 0.f && p >= cut) {
+    const uint32_t i = cand_i[lane];
     const uint4 rnd = philox4x32_10(
         make_uint4(i >> 2, static_cast<uint32_t>(row), a.offset_lo, a.offset_hi), a.seed_lo,
         a.seed_hi);
     const uint32_t w01 = i & 1 ? rnd.y : rnd.x, w23 = i & 1 ? rnd.w : rnd.z;
-    const float key = s[t] + gumbel(i & 2 ? w23 : w01);
-    if (key > best || (key == best && i < best_i)) {
+    const float key = s + gumbel(i & 2 ? w23 : w01);
+    if (key > best) {
       best = key;
       best_i = i;
     }
@@ -1375,7 +1347,8 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     return;
   }
   // Top-k: every wave finds the offsets of the segments' lists in the row's (the same values
-  // into the same words) and loads its tokens; meanwhile one wave takes a lower bound of the
+  // into the same words, and a wave's LDS operations are in order, so it can read what its own
+  // lanes wrote) and loads its tokens; meanwhile one wave takes a lower bound of the
   // k-th largest s from the segments' peaks, folded into 256 groups. The tokens that reach the
   // bound, little more than k, are kept for finish_candidates' work.
   uint32_t k = static_cast<uint32_t>(r.top_k);
@@ -1394,18 +1367,14 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     if (j < n) sh.offset[j] = total + incl - c;
     total += __shfl(incl, kWave - 1);
   }
-  bool ok = !__any(full) && total <= kRowList;  // the same in every wave
+  bool ok = !__any(full);  // the same in every wave
   if (ok) {
     // Fewer listed tokens than k: no segment had k finite logits, so every finite one is listed,
     // and the cutoff at their number keeps them all, as the row's own does.
     k = min(k, total);
-    constexpr int kOwn = kRowList / kThreads;
+    constexpr int kOwn = kRowOwn / kThreads;
     const uint2* lists = p.list + row * n * int64_t(kSegList);
-    uint2 own[kOwn];
-#pragma unroll
-    for (int t = 0; t < kOwn; ++t) {
-      const uint32_t i = tid + t * kThreads;
-      if (i >= total) break;
+    auto listed = [&](uint32_t i) {
       int lo = 0, hi = n;  // the last segment whose list starts at or before i
       while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -1414,7 +1383,14 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
         else
           hi = mid;
       }
-      own[t] = lists[lo * int64_t(kSegList) + (i - sh.offset[lo])];
+      return lists[lo * int64_t(kSegList) + (i - sh.offset[lo])];
+    };
+    uint2 own[kOwn];
+#pragma unroll
+    for (int t = 0; t < kOwn; ++t) {
+      const uint32_t i = tid + t * kThreads;
+      if (i >= total) break;
+      own[t] = listed(i);
     }
     if (warp == 0) {
       const float* peak = p.peak + row * n * kSegPeaks;
@@ -1437,34 +1413,32 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     uint32_t* cand_i = reinterpret_cast<uint32_t*>(sh.row.mass);
     float* cand_s = reinterpret_cast<float*>(cand_i + kCandidates);
     float* cand_p = cand_s + kCandidates;
+    auto keep = [&](uint2 token) {
+      const float s = __uint_as_float(token.y);
+      if (!(s >= edge)) return;
+      const uint32_t slot = atomicAdd(&sh.count, 1u);
+      if (slot < kCandidates) {
+        cand_i[slot] = token.x;
+        cand_s[slot] = s;
+      }
+    };
 #pragma unroll
     for (int t = 0; t < kOwn; ++t) {
       if (tid + t * kThreads >= total) break;
-      const float s = __uint_as_float(own[t].y);
-      if (!(s >= edge)) continue;
-      const uint32_t slot = atomicAdd(&sh.count, 1u);
-      if (slot < kCandidates) {
-        cand_i[slot] = own[t].x;
-        cand_s[slot] = s;
-      }
+      keep(own[t]);
     }
+    // A k near the lists' largest, or many segments, list more.
+    for (uint32_t i = tid + kRowOwn; i < total; i += kThreads) keep(listed(i));
     float listed_to = -FLT_MAX;
     for (int j = lane; j < n; j += kWave)
       if (seg[j].m != -INFINITY) listed_to = fmaxf(listed_to, seg[j].bound);
     listed_to = wave_max(listed_to);
     __syncthreads();
     const uint32_t kept = sh.count;
-    if (kept <= 4 * kWave) {
-      // What is left fits one wave's registers.
+    if (kept <= kWave) {
       if (warp == 0) {
-        const float inv_z = 1.f / z;
         const bool done =
-            kept <= kWave
-                ? finish_wave<1>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p, listed_to)
-            : kept <= 2 * kWave
-                ? finish_wave<2>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p, listed_to)
-                : finish_wave<4>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p,
-                                 listed_to);
+            finish_wave(a, row, cand_i, cand_s, kept, m, 1.f / z, k, r.top_p, listed_to);
         if (lane == 0) sh.ok = done;
       }
       __syncthreads();
