@@ -328,9 +328,10 @@ def _aligned16(*tensors: torch.Tensor) -> bool:
 
 def _ordinary(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may read the tensors' memory in place of a torch call that they used to
-    reach: strided, of no class or mode that takes torch's calls over, outside vmap, forward-mode
-    differentiation and tracing."""
+    reach: strided, of no class or mode that takes torch's calls over, outside autocast, vmap,
+    forward-mode differentiation and tracing."""
     return (all(t.layout == torch.strided for t in tensors)
+            and not torch.is_autocast_enabled("cuda")
             and not torch.overrides.has_torch_function(tensors)
             and torch.autograd.forward_ad._current_level < 0
             and torch._C._functorch.maybe_current_level() is None

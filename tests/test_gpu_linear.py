@@ -353,3 +353,12 @@ def test_head_linear_keeps_torch_transforms(gpu):
     out = torch.zeros(4, 16384, dtype=torch.bfloat16, device=gpu, requires_grad=True)
     with pytest.raises(RuntimeError):
         ops.head_linear(x, w, out)
+
+
+def test_head_linear_under_autocast(gpu):
+    """Autocast picks the product's type, as for torch's own call."""
+    x, w = operands(4, 16384, 128, torch.bfloat16, gpu, 31)
+    with torch.autocast("cuda", dtype=torch.float16):
+        got, want = ops.head_linear(x, w), F.linear(x, w)
+    assert got.dtype == want.dtype == torch.float16
+    assert torch.equal(got, want)
