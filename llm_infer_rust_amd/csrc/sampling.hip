@@ -236,7 +236,11 @@ __device__ __forceinline__ float candidate_edge(float s_k, float m) {
 
 // Both cutoffs and the draw among n gathered candidates (cand_p is scratch; the lists are in
 // LDS and complete: every token of the row whose p can reach the k-th largest is listed).
-// False, and nothing written, when fewer than k candidates exist. All kThreads threads call it.
+// False, and nothing written, when fewer than k candidates exist or, without MASSLESS, the k-th p
+// has no fixed-point mass under a top-p cutoff (the branch for it costs sample_row, whose search
+// finds the cutoff as well, the unrolling of its scans: 60 -> 72 us for 256 rows of 20,000 cut by
+// top-p). All kThreads threads call it.
+template <bool MASSLESS>
 __device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& a, int64_t row,
                                                   const uint32_t* cand_i, const float* cand_s,
                                                   float* cand_p, uint32_t n, float m, float inv_z,
@@ -262,7 +266,7 @@ __device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& 
   }
   __syncthreads();
   const float p_k = sh.red_f[0];
-  if (!sh.k_found) return false;
+  if (!sh.k_found || (!MASSLESS && use_p && fixed_mass(p_k) == 0)) return false;
   float cut = p_k;
   if (use_p) {
     // Mass at or above p_k; when it reaches top_p, the top-p cutoff is the largest
@@ -288,7 +292,7 @@ __device__ __forceinline__ bool finish_candidates(Shared& sh, const SampleArgs& 
       int64_t bi = 0;
       block_argmax(sh, bv, bi);
       cut = bv;
-    } else if (fixed_mass(p_k) == 0) {
+    } else if (MASSLESS && fixed_mass(p_k) == 0) {
       // Rounding kept the whole mass below the target, and all of it lies above p_k: the cutoff
       // is the lowest p that has any.
       float low = -INFINITY;
@@ -501,7 +505,8 @@ __device__ __forceinline__ void sample_row(Shared& sh, const SampleArgs& a, int6
       const uint32_t n = sh.p_lowest;
       ok = n <= kCandidates;
       if (ok) {
-        if (finish_candidates(sh, a, row, cand_i, cand_s, cand_p, n, m, inv_z, top_k, top_p))
+        if (finish_candidates<false>(sh, a, row, cand_i, cand_s, cand_p, n, m, inv_z, top_k,
+                                     top_p))
           return;
       }
     }
@@ -1226,55 +1231,91 @@ __global__ __launch_bounds__(kSegThreads) void race_segments(SampleArgs a, Split
   }
 }
 
-// finish_candidates for at most kWave candidates by one wave, each pair compared through lane
+// finish_candidates for at most 64 R candidates by one wave, each pair compared through lane
 // broadcasts: with 60 candidates 4 us against the workgroup-wide version's 16 (its LDS round
-// trips), which is the quicker one from 64 (top-k 100 of 16,385: 36.8 us a call with two to four
-// candidates a lane, 23.4 workgroup-wide). False as well when tokens that could share the k-th p
-// may not have been listed, the lists being complete down to listed_to only.
-__device__ bool finish_wave(const SampleArgs& a, int64_t row, const uint32_t* cand_i,
+// trips). False as well when tokens that could share the k-th p may not have been listed, the
+// lists being complete down to listed_to only.
+template <int R>
+__device__ __forceinline__ bool finish_wave(const SampleArgs& a, int64_t row, const uint32_t* cand_i,
                             const float* cand_s, uint32_t n, float m, float inv_z, int64_t top_k,
                             float top_p, float listed_to) {
-  const uint32_t lane = threadIdx.x % kWave;
+  const int lane = threadIdx.x % kWave;
   const bool use_p = top_p < 1.f;
   const uint32_t k = static_cast<uint32_t>(top_k);
-  const float s = lane < n ? cand_s[lane] : -INFINITY;
-  const float p = lane < n ? probability(s, m, inv_z) : -1.f;
-  const unsigned long long fx = lane < n ? fixed_mass(p) : 0ull;
-  uint32_t gt = 0, ge = 0;
-  unsigned long long mass = 0;  // at or above the own p
-  for (uint32_t u = 0; u < n; ++u) {
-    const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), u));
-    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx), u);
-    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx >> 32), u);
-    const unsigned long long f = (static_cast<unsigned long long>(hi) << 32) | lo;
-    gt += v > p;
-    ge += v >= p;
-    mass += v >= p ? f : 0ull;
+  float s[R], p[R];
+  uint32_t gt[R], ge[R];
+  unsigned long long fx[R], mass[R];  // mass at or above the own p
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const uint32_t c = lane + kWave * t;
+    s[t] = c < n ? cand_s[c] : -INFINITY;
+    p[t] = c < n ? probability(s[t], m, inv_z) : -1.f;
+    fx[t] = c < n ? fixed_mass(p[t]) : 0ull;
+    gt[t] = ge[t] = 0;
+    mass[t] = 0;
   }
-  // The k-th largest p, the mass at or above it, and the lowest s that has it.
-  const bool is_k = p >= 0.f && gt < k && ge >= k;
-  const float p_k = wave_max(is_k ? p : -1.f);
-  const bool reached = __any(is_k && mass >= mass_target(top_p));
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const int some = min(kWave, static_cast<int>(n) - kWave * t);
+    for (int u = 0; u < some; ++u) {
+      const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p[t]), u));
+      const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx[t]), u);
+      const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(fx[t] >> 32), u);
+      const unsigned long long f = (static_cast<unsigned long long>(hi) << 32) | lo;
+#pragma unroll
+      for (int w = 0; w < R; ++w) {
+        gt[w] += v > p[w];
+        const bool above = v >= p[w];
+        ge[w] += above;
+        mass[w] += above ? f : 0ull;
+      }
+    }
+  }
+  // The k-th largest p and the mass at or above it.
+  float p_k = -1.f;
+  bool reached = false;
+#pragma unroll
+  for (int t = 0; t < R; ++t)
+    if (p[t] >= 0.f && gt[t] < k && ge[t] >= k) {
+      p_k = p[t];
+      reached = mass[t] >= mass_target(top_p);
+    }
+  reached = __any(reached);
+  p_k = wave_max(p_k);
   if (p_k < 0.f) return false;
-  const float s_k = -wave_max(p == p_k ? -s : -INFINITY);
+  float s_k = INFINITY;  // the lowest s that has it
+#pragma unroll
+  for (int t = 0; t < R; ++t)
+    if (p[t] == p_k) s_k = fminf(s_k, s[t]);
+  s_k = -wave_max(-s_k);
   if (listed_to > candidate_edge(s_k, m)) return false;
   float cut = p_k;
-  if (use_p && reached)
-    cut = wave_max(p > cut && mass >= mass_target(top_p) ? p : cut);
-  else if (use_p && fixed_mass(p_k) == 0)
+  if (use_p && reached) {
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      if (p[t] > cut && mass[t] >= mass_target(top_p)) cut = p[t];
+    cut = wave_max(cut);
+  } else if (use_p && fixed_mass(p_k) == 0) {
     // Rounding kept the whole mass below the target, and all of it lies above p_k: the cutoff is
     // the lowest p that has any.
-    cut = -wave_max(fx ? -p : -INFINITY);
+    float low = INFINITY;
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      if (fx[t]) low = fminf(low, p[t]);
+    cut = -wave_max(-low);
+  }
   float best = -INFINITY;
   uint32_t best_i = static_cast<uint32_t>(a.vocab);
-  if (p > 0.f && p >= cut) {
-    const uint32_t i = cand_i[lane];
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    if (!(p[t] > 0.f && p[t] >= cut)) continue;
+    const uint32_t i = cand_i[lane + kWave * t];
     const uint4 rnd = philox4x32_10(
         make_uint4(i >> 2, static_cast<uint32_t>(row), a.offset_lo, a.offset_hi), a.seed_lo,
         a.seed_hi);
     const uint32_t w01 = i & 1 ? rnd.y : rnd.x, w23 = i & 1 ? rnd.w : rnd.z;
-    const float key = s + gumbel(i & 2 ? w23 : w01);
-    if (key > best) {
+    const float key = s[t] + gumbel(i & 2 ? w23 : w01);
+    if (key > best || (key == best && i < best_i)) {
       best = key;
       best_i = i;
     }
@@ -1435,10 +1476,17 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     listed_to = wave_max(listed_to);
     __syncthreads();
     const uint32_t kept = sh.count;
-    if (kept <= kWave) {
+    // One wave up to 64 candidates, and up to 128 under a top-p cutoff, whose masses the whole
+    // workgroup sums anew for every candidate (top-k 50 and top-p 0.9, 96 rows of 57,000, about 70
+    // candidates: 24.3 us a call with one wave, 27.8 workgroup-wide; top-k 100 of 151,936 29.6 with
+    // the workgroup, 37.7 with one wave of four candidates a lane).
+    if (kept <= kWave || (kept <= 2 * kWave && r.top_p < 1.f)) {
       if (warp == 0) {
+        const float inv_z = 1.f / z;
         const bool done =
-            finish_wave(a, row, cand_i, cand_s, kept, m, 1.f / z, k, r.top_p, listed_to);
+            kept <= kWave
+                ? finish_wave<1>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p, listed_to)
+                : finish_wave<2>(a, row, cand_i, cand_s, kept, m, inv_z, k, r.top_p, listed_to);
         if (lane == 0) sh.ok = done;
       }
       __syncthreads();
@@ -1446,8 +1494,8 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     } else {
       // The whole workgroup, where the bound itself shows the lists complete.
       ok = kept <= kCandidates && listed_to <= edge &&
-           finish_candidates(sh.row, a, row, cand_i, cand_s, cand_p, kept, m, 1.f / z, k,
-                             r.top_p);
+           finish_candidates<true>(sh.row, a, row, cand_i, cand_s, cand_p, kept, m, 1.f / z, k,
+                                   r.top_p);
     }
   }
   if (ok) return;
