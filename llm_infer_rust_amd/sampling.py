@@ -20,6 +20,7 @@ and every sampling call advances the offset by one.
 from __future__ import annotations
 
 import math
+from collections import Counter
 from dataclasses import dataclass, replace
 
 import torch
@@ -51,6 +52,43 @@ LISTED_TOP_K = 128
 # From this many rows on an all-greedy batch is quicker with one workgroup per row and one launch
 # (256 rows of 151,936: 31 us against 38; one row: 28 against 14).
 GREEDY_ROWS = 128
+# Rows that one workgroup each runs side by side, one on a CU; more take another round.
+ROUND_ROWS = 256
+
+
+def _split_pays(rows: int, vocab: int, greedy: int, race: int, listed: int, widest_k: int,
+                top_p: int, fp32: bool, vec: bool) -> bool:
+    """Whether rows spread over several workgroups beat one workgroup per row, for a batch of so
+    many greedy, unfiltered, listed top-k (the largest ``widest_k``) and top-p rows; ``vec``: every
+    row starts on 16 bytes.
+
+    The vocabulary from which it does, measured at 13 vocabularies from 16,385 to 128,256, 14 row
+    counts up to 1,024, bf16 and fp32. The split call has a launch more and a pass that grows with
+    the rows; one workgroup per row costs the same up to 256 rows and again for each further 256,
+    so that a full round needs the longest rows. Listed rows gain at every size. us, one workgroup
+    per row against split: greedy, 16 rows of 32,000 12.8 and 13.7, of 100,000 23.1 and 14.2;
+    unfiltered, 64 of 32,000 22.5 and 17.4, 256 24.1 and 28.8, 256 of 50,257, which one workgroup
+    reads token by token, 58 and 43; top-p, 256 of 32,000 78 and 104, of 80,000 144 and 122, 320 of
+    32,000 141 and 128; top-k 50 and top-p 0.9, 256 of 20,000 27.5 and 22.3. In a batch of several
+    kinds one workgroup per row waits for the slowest row and the split call for their mean (a
+    fifth top-p, 256 rows of 32,000: 82 and 58)."""
+    if greedy == rows:
+        return rows < GREEDY_ROWS and vocab >= 40_000 + 200 * rows
+    # Nine to twelve segments bound a large k loosely (k 128 of 16,385 at 256 rows: 26 and 72).
+    if widest_k > 96 and vocab < 49_152:
+        return False
+    rounds = -(-rows // ROUND_ROWS)
+    fill = (rows / (rounds * ROUND_ROWS)) ** 2
+    if top_p:
+        share = top_p / rows
+        if rounds == 1:
+            need = (97_000 if fp32 else 65_000) * share * fill
+        else:
+            need = (70_000 if fp32 else 36_000) * math.sqrt(share) * fill
+    else:
+        need = (12_000 + (60_000 if rounds == 1 else 32_000) * fill) * race / rows if vec else 0
+    return vocab >= need
+
 
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
@@ -101,7 +139,7 @@ class Sampler:
         self._param_objs: tuple | None = None
         self._params: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None
         self._top_p_rows = False  # some row of _params may be cut by top_p alone
-        self._all_greedy = False  # every row of _params takes the argmax
+        self._kinds = (0, 0, 0, 0, 0)  # _split_pays' greedy, race, listed, widest_k and top_p
         self._large_k: int | None = None  # smallest top_k of _params beyond LISTED_TOP_K
 
     def manual_seed(self, seed: int) -> None:
@@ -131,11 +169,21 @@ class Sampler:
                        torch.tensor(ps, dtype=torch.float32)), out=host)  # top-k bit for bit
             dev = host.to(device, non_blocking=True)
             self._params = (dev[:n], dev[n:2 * n].view(torch.int32), dev[2 * n:])
-            drawn = [(k, p) for t, k, p in set(zip(temps, ks, ps)) if t > 0 and p > 0]
-            large = [k for k, _ in drawn if k > LISTED_TOP_K]
-            self._top_p_rows = any(p < 1 and (k <= 0 or k > LISTED_TOP_K) for k, p in drawn)
-            self._all_greedy = not drawn
-            self._large_k = min(large, default=None)
+            greedy = race = listed = widest = top_p = 0
+            self._large_k = None
+            for (t, k, p), rows in Counter(zip(temps, ks, ps)).items():
+                if t <= 0 or p == 0:
+                    greedy += rows
+                elif 0 < k <= LISTED_TOP_K:
+                    listed += rows
+                    widest = max(widest, k)
+                else:
+                    if k > LISTED_TOP_K:
+                        self._large_k = k if self._large_k is None else min(self._large_k, k)
+                    top_p += rows if p < 1 else 0
+                    race += rows if p >= 1 else 0
+            self._top_p_rows = top_p > 0
+            self._kinds = (greedy, race, listed, widest, top_p)
             self._param_key = key
         self._param_objs = tuple(params_list)  # last: a build that raised is not taken for built
         return self._params
@@ -158,7 +206,8 @@ class Sampler:
                 top_p.data_ptr(), self.seed, self.offset, out.data_ptr())
         need = 0
         if ((self._large_k is None or self._large_k >= logits.size(1))
-                and not (self._all_greedy and rows >= GREEDY_ROWS)):
+                and _split_pays(rows, logits.size(1), *self._kinds,
+                                logits.dtype == torch.float32, logits.stride(0) % 8 == 0)):
             need = lib().mi355x_sample_workspace_bytes(rows, logits.size(1), self._top_p_rows)
         ws = None
         if need:

@@ -60,5 +60,31 @@ def test_batch_words_without_copies_of_the_parameters(pageable, monkeypatch, par
     assert torch.equal(top_p, torch.tensor([float(p.top_p) for p in normal]))
     listed = sampling.LISTED_TOP_K
     assert s._top_p_rows == any(p.top_p < 1 and not 0 < p.top_k <= listed for p in drawn)
-    assert s._all_greedy == (not drawn)
+    greedy, race, few, widest, top_p_rows = s._kinds
+    assert greedy == len(normal) - len(drawn) and greedy + race + few + top_p_rows == len(normal)
+    assert few == sum(0 < p.top_k <= listed for p in drawn)
+    assert widest == max((p.top_k for p in drawn if 0 < p.top_k <= listed), default=0)
+    assert top_p_rows == sum(p.top_p < 1 and not 0 < p.top_k <= listed for p in drawn)
     assert s._large_k == min((p.top_k for p in drawn if p.top_k > listed), default=None)
+
+
+GREEDY, RACE, TOP_K, TOP_P = (1, 0, 0, 0, 0), (0, 1, 0, 0, 0), (0, 0, 1, 50, 0), (0, 0, 0, 0, 1)
+
+
+@pytest.mark.parametrize("kind,rows,vocab,splits", [
+    (GREEDY, 1, 32000, False), (GREEDY, 1, 151936, True), (GREEDY, 64, 50257, False),
+    (GREEDY, 1, 50257, True), (GREEDY, 64, 151936, True), (GREEDY, 128, 151936, False), (RACE, 5, 32000, True),
+    (RACE, 256, 32000, False), (RACE, 256, 151936, True), (RACE, 320, 32000, True), (RACE, 256, 50257, True),
+    (TOP_K, 5, 16385, True), (TOP_K, 256, 20000, True), (TOP_K, 256, 50257, True),
+    (TOP_K, 1024, 151936, True), (TOP_P, 64, 20000, True), (TOP_P, 256, 32000, False),
+    (TOP_P, 256, 151936, True)])
+def test_batches_are_split_where_it_was_measured_quicker(kind, rows, vocab, splits):
+    greedy, race, listed, widest, top_p = kind
+    assert sampling._split_pays(rows, vocab, greedy * rows, race * rows, listed * rows, widest,
+                                top_p * rows, False, vocab % 8 == 0) == splits
+
+
+def test_a_large_listed_k_needs_many_segments():
+    assert not sampling._split_pays(5, 16385, 0, 0, 5, 128, 0, False, True)
+    assert sampling._split_pays(5, 16385, 0, 0, 5, 96, 0, False, True)
+    assert sampling._split_pays(5, 151936, 0, 0, 5, 128, 0, False, True)
