@@ -536,8 +536,10 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // rows at one row: K 4096 64 x 64 tiles 192 us, 64 x 128 tiles 235; K 5120 239 and 236); each
 // further M tile takes part of that again from L2. x is re-read per N tile at about 80 TB/s, which
 // tells tile widths apart under a large head. Split-K partials are written, and read by the pass that
-// follows, at about 4.2 TB/s, with 0.6 us and 0.3 per split besides. 3 us of launch and latency do
-// not depend on the choice.
+// follows, at about 4.2 TB/s, with 0.6 us and 0.3 per split besides, or 0.1 for few rows of a
+// narrow output, whose norm pass has them all in flight at once (1024 x 2048 with its norm at 45
+// rows 8.0 us with 4 splits, 7.4 with 8; 576 x 1536 at one 6.3 and 5.7; 2048 x 6144 at 96 rows
+// 14.0 and 14.6). 3 us of launch and latency do not depend on the choice.
 // Fitted to every tiling of 25 shapes (hidden 1024 to 8192, K 576 to 18944) at 18 row counts from
 // 1 to 256, alone and with the norm pass, and of 23 heads at up to 64 rows: the tiling it picks
 // takes 0.5% longer than the fastest measured on average and 16% at worst, and its own figure is
@@ -554,7 +556,9 @@ double estimate(const TileConfig& t, int splits, int64_t M, int64_t N, int64_t K
   const double weights = double(N) * double(K) * 2 / stream * (1. + 0.6 * double(tiles_m - 1));
   const double x_reads = double(blocks) * double(std::min<int64_t>(M, t.bm)) * k_bytes / 80e6;
   const double partials =
-      splits > 1 ? double(splits) * double(M) * double(N) * 8 / 4.2e6 + 0.6 + 0.3 * splits : 0.;
+      splits > 1 ? double(splits) * double(M) * double(N) * 8 / 4.2e6 + 0.6 +
+                       (M <= 64 && N <= 2048 ? 0.1 : 0.3) * splits
+                 : 0.;
   return 3. + std::max(rounds * double(t.bm + t.bn) * k_bytes / 50e3, weights) + x_reads +
          partials;
 }

@@ -134,7 +134,8 @@ def test_linear_workspace_bytes_query(native):
 
 @pytest.mark.parametrize("m,n,k,splits", [(65, 4096, 4096, 4), (96, 3072, 3072, 4),
                                           (1, 151936, 2048, 1), (8, 151936, 4096, 1),
-                                          (144, 6144, 2560, 2)])
+                                          (144, 6144, 2560, 2), (45, 1024, 2048, 8),
+                                          (1, 576, 1536, 8), (65, 1024, 2048, 4)])
 def test_linear_splits_no_more_than_pays(native, m, n, k, splits):
     """K splits where more of them were measured slower on 256 compute units (the head of 151,936
     rows and K 2048 at one row: 104 us unsplit, 136 with two)."""
