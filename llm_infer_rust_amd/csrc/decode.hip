@@ -1533,8 +1533,9 @@ extern "C" void* mi355x_decode_prepare(void* existing, const int32_t* block_tabl
                                       (plan->host_lengths[r] + page_size - 1) / page_size);
     int64_t chunk = 0, wgs = 0;
     const int64_t items = schedule(plan->host_lengths.data(), batch, shape.workgroups,
-                                   shape.max_item, shape.tile, graph, host + layout.o_work, items_cap,
-                                   host + layout.o_merge, &chunk, host + layout.o_wg, wg_cap, &wgs);
+                                   shape.max_item, shape.tile, graph, host + layout.o_work,
+                                   items_cap, host + layout.o_merge, &chunk, host + layout.o_wg,
+                                   wg_cap, &wgs);
     if (items < 0) {
       set_error("decode work list exceeds its capacity");
       return nullptr;

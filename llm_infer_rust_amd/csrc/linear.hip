@@ -145,7 +145,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void linear_kernel(LinearArgs a) {
   // First K step of this workgroup (the others follow cyclically). With every workgroup at
   // the same step, the rows' 128-byte chunks lie a row stride apart (8 KB at K 4096) and meet
   // in a subset of the memory channels; one step apart per N tile they spread over all of
-  // them: gate_up 24576 x 4096 at 24 rows 41.9 -> 35.3 us, 8192 x 8192 with its norm at 24 rows
+  // them: gate_up 24576 x 4096 at 24 rows 40.8 -> 33.4 us, 8192 x 8192 with its norm at 24 rows
   // 36.0 -> 29.5 and at 192 rows 51.5 -> 49.9. Where several M tiles re-read x from L2 and K is
   // at most 4096 the phases are eight, an eighth of K apart, so that more of the tiles in flight
   // read the same x chunks: gate_up at 256 rows 62.1 us against 64.4 with a phase per tile;
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void linear_kernel(LinearArgs a) {
     kt = a.tiles_m == 1 || a.K > 4096 ? phase % n_k : (phase & 7) * n_k / 8;
   }
   // Weights that are read once are copied non-temporally and leave L2 to x (gate_up at 24 rows
-  // 38.8 -> 35.3 us); keep_weights is the host's word that several M tiles read them from L2. It
+  // 36.7 -> 33.4 us); keep_weights is the host's word that several M tiles read them from L2. It
   // is asked once, outside the K loop (gate_up 6144 x 1024 at one row 7.9 us with the question at
   // every copy, 7.4 so).
   auto issue = [&](int stage, auto keep) {
@@ -535,8 +535,8 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // that every workgroup starts at the same K step of rows a power of two apart (the head of 151,936
 // rows at one row: K 4096 64 x 64 tiles 192 us, 64 x 128 tiles 235; K 5120 239 and 236); each
 // further M tile takes part of that again from L2. x is re-read per N tile at about 80 TB/s, which
-// tells tile widths apart under a large head. Split-K partials are written, and read by the pass that
-// follows, at about 4.2 TB/s, with 0.6 us and 0.3 per split besides, or 0.1 for few rows of a
+// tells tile widths apart under a large head. Split-K partials are written, and read by the pass
+// that follows, at about 4.2 TB/s, with 0.6 us and 0.3 per split besides, or 0.1 for few rows of a
 // narrow output, whose norm pass has them all in flight at once (1024 x 2048 with its norm at 45
 // rows 8.0 us with 4 splits, 7.4 with 8; 576 x 1536 at one 6.3 and 5.7; 2048 x 6144 at 96 rows
 // 14.0 and 14.6). 3 us of launch and latency do not depend on the choice.
@@ -804,7 +804,8 @@ extern "C" const char* mi355x_linear_add_rms_norm(const void* x, int64_t ldx, co
                                                   void* workspace, int64_t workspace_bytes,
                                                   int32_t cus, int64_t dtype, void* stream) {
   return linear_add_rms_norm(x, ldx, w, ldw, residual, ldr, norm_weight, eps, out, ldo, M, N, K,
-                             workspace, workspace_bytes, cus, dtype, 129, 1024, "1032..8192", stream);
+                             workspace, workspace_bytes, cus, dtype, 129, 1024, "1032..8192",
+                             stream);
 }
 
 extern "C" const char* mi355x_linear_add_rms_norm_narrow(const void* x, int64_t ldx, const void* w,

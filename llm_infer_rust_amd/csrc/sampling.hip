@@ -1,4 +1,5 @@
-// Joint top-k / top-p token sampling for gfx950, one workgroup per logits row.
+// Joint top-k / top-p token sampling for gfx950: one workgroup per logits row (the algorithm
+// below), or a row spread over several (further down).
 //
 // Semantics (src/engine/sampling.rs:239-269, 330-372, 409-428):
 //   * parameters are normalised as SamplingParams::normalized does: a top_p
@@ -625,8 +626,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
 // rows and walks a row two to five times; here every workgroup holds one segment of a row in
 // registers, so the logits are read once for greedy, unfiltered and top-k rows. Bound by
 // VALU work where the rows are many (an exponential per logit; 256 rows of 151,936 bf16 logits,
-// top-k 50 and top-p 0.9: 26 + 16 us a call against 66 with one workgroup per row), by latency
-// and launches where they are few (5 mixed rows 197 -> 50 us, 5 top-k rows 72 -> 23):
+// top-k 50 and top-p 0.9: 37 us a call, 26 + 11 traced, against 66 with one workgroup per row), by
+// latency and launches where they are few (5 mixed rows 193 -> 41 us, 5 top-k rows 56 -> 21):
 //   sample_segments  per segment: the argmax, or the race's best token, or the segment's max
 //                    and sum of exp(s - max); top-k rows also list the tokens at or above a
 //                    bound on the segment's k-th largest (the k-th largest of the 256 threads'
@@ -640,7 +641,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
 //                    ties) or whose parameters fit none of the above take sample_row. Rows with
 //                    fewer than k finite logits (a grammar's mask) and rows whose k-th p has no
 //                    fixed-point mass (sharp logits) are joined too: 5 rows of 151,936 with 30
-//                    tokens allowed 95 -> 21 us, with logits of deviation 25 286 -> 25.
+//                    tokens allowed 95 us when walked whole after the segments, 16 joined, with
+//                    logits of deviation 25 283 and 21.
 // Cutoffs and draws are sample_row's: masses are the same fixed-point sums, the race is the
 // same, and the sum of exp differs by its fp32 rounding only.
 // ---------------------------------------------------------------------------
@@ -1478,8 +1480,8 @@ __global__ __launch_bounds__(kThreads) void sample_finish(SampleArgs a, SplitArg
     const uint32_t kept = sh.count;
     // One wave up to 64 candidates, and up to 128 under a top-p cutoff, whose masses the whole
     // workgroup sums anew for every candidate (top-k 50 and top-p 0.9, 96 rows of 57,000, about 70
-    // candidates: 24.3 us a call with one wave, 27.8 workgroup-wide; top-k 100 of 151,936 29.6 with
-    // the workgroup, 37.7 with one wave of four candidates a lane).
+    // candidates: 24.3 us a call with one wave, 27.8 workgroup-wide; top-k 100 of one row of
+    // 151,936 29.6 with the workgroup, 37.7 with one wave of four candidates a lane).
     if (kept <= kWave || (kept <= 2 * kWave && r.top_p < 1.f)) {
       if (warp == 0) {
         const float inv_z = 1.f / z;
@@ -1620,8 +1622,8 @@ extern "C" int64_t mi355x_sample_workspace_bytes(int64_t rows, int64_t vocab, bo
   if (rows <= 0 || vocab <= 0 || vocab >= (int64_t(1) << 32)) return 0;
   const int64_t n = rows * split_plan(rows, vocab).segments;
   if (n == 0) return 0;
-  return round256(n * int64_t(sizeof(Segment))) + n * kSegPeaks * 4 + n * kSegList * int64_t(sizeof(uint2)) +
-         round256(rows * 4 * int64_t(sizeof(LevelState))) +
+  return round256(n * int64_t(sizeof(Segment))) + n * kSegPeaks * 4 +
+         n * kSegList * int64_t(sizeof(uint2)) + round256(rows * 4 * int64_t(sizeof(LevelState))) +
          (top_p_rows ? rows * kHistWords * 8 : 0);
 }
 

@@ -353,8 +353,9 @@ def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.T
                         eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """``y = linear(x, weight)`` then ``add_rms_norm(y, residual, norm_weight, eps)``,
     returning ``(normed, residual)`` with ``residual`` updated in place. Decode-sized
-    products run as one projection plus one fused reduce/residual/norm pass (bit-identical
-    to the two separate steps); everything else runs the two steps."""
+    products run as one projection plus one fused reduce/residual/norm pass (bit-identical to
+    ``decode_linear`` then ``add_rms_norm``, also for the few rows of a long K that ``linear``
+    leaves to hipBLASLt, whose sums run in another order); everything else runs the two steps."""
     m, k = (x.shape if x.dim() == 2 else (0, 0))
     n = weight.size(0)
     if (x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and weight.is_contiguous()
@@ -395,8 +396,9 @@ def uses_silu_kernel(rows: int, width: int, k: int) -> bool:
 def decode_linear_silu_mul(x: torch.Tensor, weight: torch.Tensor,
                            out: torch.Tensor | None = None, config: int = -1) -> torch.Tensor:
     """``silu_and_mul(x @ weight.T)`` in one gfx950 launch: weight ``[2 W, K]`` (gate rows,
-    then up rows), result ``[M, W]``, bit-identical to ``decode_linear`` (unsplit) followed
-    by ``silu_and_mul``."""
+    then up rows), result ``[M, W]``, bit-identical to ``decode_linear`` with the same tiling
+    and one split followed by ``silu_and_mul`` (another tile width, or another number of row
+    tiles, sums K in another order)."""
     _require_device(x, "decode_linear_silu_mul")
     dt = dtype_code(x)
     if (x.dim() != 2 or weight.dim() != 2 or x.stride(1) != 1 or not weight.is_contiguous()

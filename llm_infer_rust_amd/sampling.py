@@ -49,8 +49,10 @@ class SamplingParams:
 # larger one below the vocabulary takes one workgroup per row from the start (k 200, 64 rows of
 # 151,936: 61 us; as a fallback within the split call 92).
 LISTED_TOP_K = 128
-# From this many rows on an all-greedy batch is quicker with one workgroup per row and one launch
-# (256 rows of 151,936: 31 us against 38; one row: 28 against 14).
+# From this many rows on an all-greedy batch takes one workgroup per row and one launch: what the
+# split call still gives there is small below 100,000 columns (127 fp32 rows of 80,000: 3%) and gone
+# in a full round (151,936 columns, one workgroup per row against split: one row 28.6 us and 11.5,
+# 128 rows 32.2 and 23.9, 256 rows 33.0 and 34.9).
 GREEDY_ROWS = 128
 # Rows that one workgroup each runs side by side, one on a CU; more take another round.
 ROUND_ROWS = 256
