@@ -248,7 +248,8 @@ def test_silu_mul_matches_oracle(gpu, dtype, tokens, width):
     within_one_ulp(got, want, dtype)
 
 
-@pytest.mark.parametrize("tokens,width", [(1864135, 24), (1864136, 24), (701, 65544)])
+@pytest.mark.parametrize("tokens,width", [(1864135, 24), (1864136, 24), (701, 65544),
+                                          (2796202, 24), (2796203, 24), (1025, 65544)])
 def test_silu_mul_large_launch_equals_row_blocks(gpu, tokens, width):
     """Either side of the size from which the pass is non-temporal, with a partly filled last
     workgroup: the same words as the rows in smaller launches."""

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 import torch
 
+from llm_infer_rust_amd import sampling
 from llm_infer_rust_amd._native import lib
 from llm_infer_rust_amd.sampling import Sampler, SamplingError, SamplingParams
 from oracle import bf16 as obf
@@ -205,6 +206,12 @@ def test_top_k_candidate_path_edges_match_oracle(gpu, dtype, name, case, k, p):
 ROW_KINDS = [sp(), sp(0.7, 50, 0.9), sp(1.0), sp(1.3, -1, 0.6), sp(0.8, 128), sp(0.5, 5, 0.3)]
 
 
+@pytest.fixture
+def split(monkeypatch):
+    """Every batch that can be split is, also where one workgroup per row is the quicker one."""
+    monkeypatch.setattr(sampling, "_split_pays", lambda *args: True)
+
+
 def one_workgroup_per_row(logits, params, seed, offset):
     """mi355x_sample on the parameter arrays the sampler itself would pass."""
     s = Sampler(seed)
@@ -221,7 +228,7 @@ def one_workgroup_per_row(logits, params, seed, offset):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("rows,vocab", [(6, 16384), (7, 16385), (8, 18432), (21, 30001),
                                         (40, 65539), (140, 70000), (300, 20000), (60, 151936)])
-def test_split_rows_equal_one_workgroup_per_row(gpu, dtype, rows, vocab):
+def test_split_rows_equal_one_workgroup_per_row(gpu, split, dtype, rows, vocab):
     """Nine and more segments per row, 1, 2 and 4 chunks per segment, rows that end inside a
     chunk, every kind of row in one call. Equal ids: the two differ by the fp32 rounding of the
     exponentials' sum only."""
@@ -235,7 +242,7 @@ def test_split_rows_equal_one_workgroup_per_row(gpu, dtype, rows, vocab):
     assert (lib().mi355x_sample_workspace_bytes(rows, vocab, True) == 0) == (vocab <= 16384)
 
 
-def test_large_top_k_takes_one_workgroup_per_row(gpu):
+def test_large_top_k_takes_one_workgroup_per_row(gpu, split):
     """A top_k past the lists: routed whole by the sampler, and correct inside a split call."""
     logits = (torch.randn(6, 30000, generator=torch.Generator().manual_seed(4)) * 3).to(gpu)
     params = [sp(0.9, 129, 0.8), sp(0.7, 50, 0.9), sp(), sp(1.0, 5000), sp(0.9, -1, 0.5), sp(1.0)]
@@ -250,7 +257,7 @@ def test_large_top_k_takes_one_workgroup_per_row(gpu):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("case", ["equal", "coarse", "few", "empty_segment", "sorted", "nan", "inf",
                                   "all_hidden"])
-def test_split_rows_on_awkward_distributions(gpu, dtype, case):
+def test_split_rows_on_awkward_distributions(gpu, split, dtype, case):
     """Lists that overflow (ties), fewer finite logits than k, segments without a finite logit,
     every large logit in one segment, and invalid values in one segment only."""
     rows, vocab = 2 * len(ROW_KINDS), 50000
@@ -296,7 +303,7 @@ def test_split_workspace_is_checked(gpu):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("allowed", [1, 4, 30, 49, 50, 51, 127, 128, 300])
 @pytest.mark.parametrize("spread", [1.0, 10.0, 40.0])
-def test_split_rows_with_few_or_negligible_tokens(gpu, dtype, allowed, spread):
+def test_split_rows_with_few_or_negligible_tokens(gpu, split, dtype, allowed, spread):
     """Fewer finite logits than k, as many and a few more, spread over the row or side by side,
     with a k-th probability that does or does not reach the fixed-point mass; masks of -inf and of
     the type's lowest value. Equal ids with one workgroup per row."""
@@ -319,7 +326,7 @@ def test_split_rows_with_few_or_negligible_tokens(gpu, dtype, allowed, spread):
     assert torch.equal(got, one_workgroup_per_row(logits, params, allowed, 0))
 
 
-def test_sampling_without_room_for_the_split_workspace(gpu, monkeypatch):
+def test_sampling_without_room_for_the_split_workspace(gpu, split, monkeypatch):
     """A batch that was sampled before rows were split is still sampled when there is no memory
     left for the split call's workspace."""
     g = torch.Generator().manual_seed(40)
@@ -337,3 +344,28 @@ def test_sampling_without_room_for_the_split_workspace(gpu, monkeypatch):
         got = s.sample_batch_device(logits, ROW_KINDS)
     assert s.offset == 1
     assert torch.equal(got, one_workgroup_per_row(logits, ROW_KINDS, 3, 0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [16385, 34817, 151936, 256000])
+@pytest.mark.parametrize("spread", [3.0, 40.0])
+def test_split_rows_with_long_lists_and_wide_cutoffs(gpu, split, dtype, vocab, spread):
+    """A k up to the lists' largest: more listed tokens in a row than are loaded before its bound is
+    known (k 64 of 256,000 and 100 of 151,936 and up), 64 candidates and either side, and k-th
+    probabilities without fixed-point mass. Equal ids with one workgroup per row."""
+    params = [sp(0.8, k, p) for k in (40, 56, 60, 64, 65, 80, 100, 127, 128)
+              for p in (1.0, 0.9, 0.3)]
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    logits = (torch.empty(len(params), vocab, device=gpu).normal_(generator=g) * spread).to(dtype)
+    got = Sampler(7).sample_batch_device(logits, params)
+    assert torch.equal(got, one_workgroup_per_row(logits, params, 7, 0))
+
+
+@pytest.mark.parametrize("rows,vocab,params", [
+    (16, 32000, sp()), (16, 65536, sp()), (256, 32000, sp(1.0)), (32, 32000, sp(1.0)),
+    (256, 20000, sp(1.0, -1, 0.9)), (16, 20000, sp(1.0, -1, 0.9)), (5, 20000, sp(1.0, 100))])
+def test_either_route_gives_the_same_ids(gpu, rows, vocab, params):
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    logits = torch.empty(rows, vocab, device=gpu).normal_(generator=g).to(torch.bfloat16)
+    got = Sampler(8).sample_batch_device(logits, [params] * rows)
+    assert torch.equal(got, one_workgroup_per_row(logits, [params] * rows, 8, 0))
