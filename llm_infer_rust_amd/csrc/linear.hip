@@ -580,7 +580,10 @@ constexpr int64_t kMaxPartialBytes = int64_t(32) << 20;
 // The tiling with the least estimate. K is split further only while the tiles leave less than two
 // rounds of workgroups, and 128 x 192 tiles keep 16 K steps (with fewer, filling their three
 // stages is not worth it: QKV 6144 x 2560 at 144 rows 22.3 us with 128 x 128 tiles and 2 splits,
-// 23.5 with 128 x 192 and 4).
+// 23.5 with 128 x 192 and 4). For up to 64 rows they take one round at most, where they come near
+// the others' rate with the fewest bytes a CU; in the rounds of a head, one workgroup a CU with half
+// its rows empty, they do not (one row, 64 x 128 tiles against 128 x 192: 152,064 x 3584 162 and
+// 199 us, 128,256 x 4096 153 and 179).
 Choice choose(int64_t M, int64_t N, int64_t K, int cus) {
   Choice best{7, 1};
   double best_us = 1e30;
@@ -590,7 +593,7 @@ Choice choose(int64_t M, int64_t N, int64_t K, int cus) {
     for (int s = 1; s <= 8 && K % (int64_t(s) * kBK) == 0; s *= 2) {
       if (s > 1 && (int64_t(s) * M * N * 4 > kMaxPartialBytes || tiles * s >= 4 * int64_t(cus)))
         break;
-      if (c == 0 && K / s < 16 * kBK) break;
+      if (c == 0 && (K / s < 16 * kBK || (M <= 64 && tiles * s > cus))) break;
       const double us = estimate(t, s, M, N, K, cus);
       if (us < best_us) {
         best = {c, s};

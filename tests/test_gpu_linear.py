@@ -362,3 +362,13 @@ def test_head_linear_under_autocast(gpu):
         got, want = ops.head_linear(x, w), F.linear(x, w)
     assert got.dtype == want.dtype == torch.float16
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m", [1, 64])
+def test_head_takes_narrow_tiles(gpu, m):
+    """A head of several rounds of workgroups and few rows runs on 64 x 128 tiles: the bits, which
+    follow a tiling's own K order, are theirs and not those of 128 x 192."""
+    x, w = operands(m, 98304, 1152, torch.bfloat16, gpu, 98304)
+    got = ops.decode_linear(x, w)
+    assert torch.equal(got, ops.decode_linear(x, w, config=7, splits=1))
+    assert not torch.equal(got, ops.decode_linear(x, w, config=0, splits=1))
