@@ -430,19 +430,21 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 # The head's product (more columns than the layer products) of up to this many rows goes to the
-# gfx950 kernel: 151,936 x 4096 at 1 / 24 / 64 rows 194 / 205 / 231 us (6.4 TB/s of weights at
-# one row) against 249 / 272 / 273 on hipBLASLt, which is quicker from 96 rows (274 against
-# 280); 151,936 x 1024 51 / 57 / 69 against 59 / 70 / 83. A wide row whose length is no power of
-# two suits hipBLASLt, whose reads then spread over the memory channels: 152,064 x 5120 at
-# 8 / 32 / 48 / 64 rows 294 / 304 / 310 / 318 us here, 318 / 345 / 290 / 311 there, 152,064 x 3584
-# 207 / 214 / 217 / 222 and 242 / 265 / 207 / 206. K of 3072 and less is quicker here, or within
-# the 5% that two runs differ by, up to 64 rows (24 vocabularies from 8,196 to 256,000).
+# gfx950 kernel: 151,936 x 4096 at 1 / 24 / 64 rows 188 / 198 / 249 us (6.6 TB/s of weights at
+# one row) against 242 / 260 / 258 on hipBLASLt, which is quicker from 96 rows (274 against
+# 280); 151,936 x 1024 50 / 55 / 71 against 60 / 71 / 80. A wide row whose length is no power of
+# two suits hipBLASLt, whose reads then spread over the memory channels: 100,352 x 5120 at 8 / 32 /
+# 48 / 64 rows 177 / 195 / 208 / 219 us here, 213 / 240 / 187 / 218 there, 262,144 x 3840 299 / 339 /
+# 369 / 396 and 325 / 348 / 354 / 360; likewise the largest heads of shorter rows, 262,144 x 2560 at
+# 24 / 48 / 64 rows 229 / 271 / 286 and 234 / 248 / 256, while 200,000 x 2560 at 64 rows takes 223 and
+# 237, and 151,936 x 2560 at 64 rows 164 and 177.
 HEAD_MAX_ROWS = 64
 HEAD_MAX_ROWS_WIDE = 32
 
 
-def _head_rows(k: int) -> int:
-    return HEAD_MAX_ROWS if k <= 3072 or k & (k - 1) == 0 else HEAD_MAX_ROWS_WIDE
+def _head_rows(n: int, k: int) -> int:
+    short = k <= 3072 and n * k <= 550_000_000
+    return HEAD_MAX_ROWS if short or k & (k - 1) == 0 else HEAD_MAX_ROWS_WIDE
 
 
 def head_linear(x: torch.Tensor, weight: torch.Tensor,
@@ -453,7 +455,7 @@ def head_linear(x: torch.Tensor, weight: torch.Tensor,
         x.requires_grad or weight.requires_grad or (out is not None and out.requires_grad))
     if (not wants_grad and _ordinary(x, weight) and x.is_cuda and x.dim() == 2
             and weight.dim() == 2
-            and 0 < x.size(0) <= _head_rows(x.size(1))
+            and 0 < x.size(0) <= _head_rows(weight.size(0), x.size(1))
             and weight.size(0) > DECODE_MAX_N and weight.size(0) % 4 == 0
             and x.size(1) > 0 and x.size(1) % 64 == 0 and weight.size(1) == x.size(1)
             and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype
