@@ -64,6 +64,7 @@ struct LinearArgs {
   int32_t splits, k_per_split;  // k_per_split is a multiple of kBK
   int32_t tiles_m, tiles_n, groups;  // groups = tiles_n * splits rounded up to 8
   int32_t keep_weights;              // the weight copies are plain ones
+  int32_t phases;                    // start steps of the N tiles: 0 one, 1 one per tile, 8 eight
 };
 
 // Swizzled position of 16-byte chunk c in tile row r: c ^ f(r) with
@@ -146,17 +147,14 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void linear_kernel(LinearArgs a) {
   // the same step, the rows' 128-byte chunks lie a row stride apart (8 KB at K 4096) and meet
   // in a subset of the memory channels; one step apart per N tile they spread over all of
   // them: gate_up 24576 x 4096 at 24 rows 40.8 -> 33.4 us, 8192 x 8192 with its norm at 24 rows
-  // 36.0 -> 29.5 and at 192 rows 51.5 -> 49.9. Where several M tiles re-read x from L2 and K is
-  // at most 4096 the phases are eight, an eighth of K apart, so that more of the tiles in flight
-  // read the same x chunks: gate_up at 256 rows 62.1 us against 64.4 with a phase per tile;
-  // at K 8192 eight phases meet again (8192 x 8192 at 192 rows 59.9 us). The phase depends on
-  // the tile modulo half the tiles, and a SILU tile's on its pair, so with the same tile shape
-  // gate column j, up column j and their fused tile sum K in one order; where N / 2 ends inside
-  // a tile that cannot hold and every tile starts at 0.
+  // 36.0 -> 29.5 and at 192 rows 51.5 -> 49.9. How many start steps there are is k_phases' choice.
+  // The phase depends on the tile modulo half the tiles, and a SILU tile's on its pair, so with the
+  // same tile shape gate column j, up column j and their fused tile sum K in one order; where N / 2
+  // ends inside a tile that cannot hold and every tile starts at 0.
   int kt = 0;
-  if ((a.N / 2) % BN == 0) {
+  if (a.phases && (a.N / 2) % BN == 0) {
     const int phase = SILU ? tn >> 1 : tn % (a.tiles_n >> 1);
-    kt = a.tiles_m == 1 || a.K > 4096 ? phase % n_k : (phase & 7) * n_k / 8;
+    kt = a.phases == 1 ? phase % n_k : (phase & 7) * n_k / 8;
   }
   // Weights that are read once are copied non-temporally and leave L2 to x (gate_up at 24 rows
   // 36.7 -> 33.4 us); keep_weights is the host's word that several M tiles read them from L2. It
@@ -574,6 +572,18 @@ bool keeps_weights(const TileConfig& t, int64_t M, int64_t N, int64_t K) {
   return M > t.bm && ((M - 1) % t.bm < t.bm / 4 || N * K * 2 <= (int64_t(32) << 20));
 }
 
+// Start steps of the N tiles (LinearArgs::phases). One row tile, or K above 4096: one per tile. Where
+// several row tiles re-read x from L2 and K is at most 4096 the phases are eight, an eighth of K
+// apart, so that more of the tiles in flight read the same x chunks (gate_up 24576 x 4096 at 256 rows
+// 62.1 us against 64.4 with a phase per tile; at K 8192 eight phases meet again, 8192 x 8192 at 192
+// rows 59.9 us). Rows above 2048 long of up to 32 MiB of weights are better read together: the row
+// tiles find them in L2 either way (4096 x 4096 with its norm at 96 / 128 / 256 rows 16.1 / 17.2 /
+// 22.6 us, with eight phases 16.6 / 17.8 / 23.1; gate_up 8192 x 2048 at 256 rows 17.9 and 17.6).
+int k_phases(int64_t tiles_m, int64_t N, int64_t K) {
+  if (tiles_m == 1 || K > 4096) return 1;
+  return K > 2048 && N * K * 2 <= (int64_t(32) << 20) ? 0 : 8;
+}
+
 // Partials the library may choose to write: what the allocation-free entry's scratch holds.
 constexpr int64_t kMaxPartialBytes = int64_t(32) << 20;
 
@@ -673,6 +683,7 @@ const char* run_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, v
   a.tiles_n = static_cast<int32_t>(ceil_div(N, t.bn));
   a.groups = static_cast<int32_t>(ceil_div(int64_t(a.tiles_n) * a.splits, 8) * 8);
   a.keep_weights = keeps_weights(t, M, N, K);
+  a.phases = k_phases(a.tiles_m, N, K);
   const int64_t blocks = int64_t(a.groups) * a.tiles_m;
   if (blocks > (int64_t(1) << 31) - 1) return set_error("mi355x_linear: grid too large");
   if (dtype == 0)
@@ -852,6 +863,7 @@ extern "C" const char* mi355x_linear_silu_mul(const void* x, int64_t ldx, const 
   a.tiles_n = static_cast<int32_t>(ceil_div(N, t.bn));
   a.groups = static_cast<int32_t>(ceil_div(a.tiles_n, 8) * 8);
   a.keep_weights = keeps_weights(t, M, N, K);
+  a.phases = k_phases(a.tiles_m, N, K);
   const int64_t blocks = int64_t(a.groups) * a.tiles_m;
   if (blocks > (int64_t(1) << 31) - 1) return set_error("mi355x_linear_silu_mul: grid too large");
   auto s = static_cast<hipStream_t>(stream);
