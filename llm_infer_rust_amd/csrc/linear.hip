@@ -561,15 +561,22 @@ double estimate(const TileConfig& t, int splits, int64_t M, int64_t N, int64_t K
          partials;
 }
 
-// Whether the weights' copies are plain instead of non-temporal. Several M tiles read each weight
-// tile, and L2 serves all but the first reader only while they run in step. They part where the
-// last M tile is nearly empty (its x rows are one row repeated, so it waits less): 5120 x 17408
-// with its norm at 129 / 144 / 160 rows 76 / 75 / 68 us non-temporal, 63 / 66 / 69 plain, 4096 x
-// 12288 at 72 rows 33.3 and 30.8. Up to 32 MiB of weights plain copies are quicker for any last
-// tile (4096 x 4096 at 192 rows 22.5 and 21.1); above it they cost (8192 x 8192 at 224 rows 51.9
-// and 54.4, 4096 x 12288 at 208 rows 41.7 and 43.7).
-bool keeps_weights(const TileConfig& t, int64_t M, int64_t N, int64_t K) {
-  return M > t.bm && ((M - 1) % t.bm < t.bm / 4 || N * K * 2 <= (int64_t(32) << 20));
+// Whether the weights' copies are plain instead of non-temporal. Several row tiles read each weight
+// tile, and L2 serves all but the first reader only while they run in step. They part where the last
+// of 128-row tiles is nearly empty (its x rows are one row repeated, so it waits less): 5120 x 17408
+// with its norm at 129 rows 69.0 us non-temporal, 67.0 plain, 4096 x 12288 41.0 and 38.2, gate_up
+// 34816 x 5120 144 and 130; 64-row tiles lose by it (gate_up 12288 x 2048 at 72 rows 16.2 and 17.1,
+// 2048 x 6144 with its norm at 65 rows 13.0 and 13.6). Up to 32 MiB of weights plain copies are
+// quicker for fuller last tiles as well (4096 x 4096 with its norm at 192 rows 21.2 and 20.4, 1024 x
+// 3072 10.3 and 9.7), but not for a gate_up (12288 x 1024 at 128 rows 10.8 and 11.5) nor, above
+// 16 MiB, for a K of 8192 and more (1536 x 8960 at 128 rows 17.0 and 17.3); above 32 MiB they cost
+// (8192 x 8192 at 224 rows 51.9 and 54.4, 4096 x 12288 at 208 rows 41.7 and 43.7).
+bool keeps_weights(const TileConfig& t, int64_t M, int64_t N, int64_t K, bool silu) {
+  if (M <= t.bm) return false;
+  const bool nearly_empty = (M - 1) % t.bm < t.bm / 4;
+  if (nearly_empty) return t.bm == 128;
+  const int64_t bytes = N * K * 2;
+  return !silu && bytes <= (int64_t(32) << 20) && (K < 8192 || bytes <= (int64_t(16) << 20));
 }
 
 // Start steps of the N tiles (LinearArgs::phases). One row tile, or K above 4096: one per tile. Where
@@ -682,7 +689,7 @@ const char* run_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, v
   a.tiles_m = static_cast<int32_t>(ceil_div(M, t.bm));
   a.tiles_n = static_cast<int32_t>(ceil_div(N, t.bn));
   a.groups = static_cast<int32_t>(ceil_div(int64_t(a.tiles_n) * a.splits, 8) * 8);
-  a.keep_weights = keeps_weights(t, M, N, K);
+  a.keep_weights = keeps_weights(t, M, N, K, false);
   a.phases = k_phases(a.tiles_m, N, K);
   const int64_t blocks = int64_t(a.groups) * a.tiles_m;
   if (blocks > (int64_t(1) << 31) - 1) return set_error("mi355x_linear: grid too large");
@@ -862,7 +869,7 @@ extern "C" const char* mi355x_linear_silu_mul(const void* x, int64_t ldx, const 
   a.tiles_m = static_cast<int32_t>(ceil_div(M, t.bm));
   a.tiles_n = static_cast<int32_t>(ceil_div(N, t.bn));
   a.groups = static_cast<int32_t>(ceil_div(a.tiles_n, 8) * 8);
-  a.keep_weights = keeps_weights(t, M, N, K);
+  a.keep_weights = keeps_weights(t, M, N, K, true);
   a.phases = k_phases(a.tiles_m, N, K);
   const int64_t blocks = int64_t(a.groups) * a.tiles_m;
   if (blocks > (int64_t(1) << 31) - 1) return set_error("mi355x_linear_silu_mul: grid too large");
