@@ -626,8 +626,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a, bool vec
 // rows and walks a row two to five times; here every workgroup holds one segment of a row in
 // registers, so the logits are read once for greedy, unfiltered and top-k rows. Bound by
 // VALU work where the rows are many (an exponential per logit; 256 rows of 151,936 bf16 logits,
-// top-k 50 and top-p 0.9: 37 us a call, 26 + 11 traced, against 66 with one workgroup per row), by
-// latency and launches where they are few (5 mixed rows 193 -> 41 us, 5 top-k rows 56 -> 21):
+// top-k 50 and top-p 0.9: 37 us a call, 26 + 11 traced, against 65 with one workgroup per row), by
+// latency and launches where they are few (5 mixed rows 209 -> 42 us, 5 top-k rows 56 -> 21):
 //   sample_segments  per segment: the argmax, or the race's best token, or the segment's max
 //                    and sum of exp(s - max); top-k rows also list the tokens at or above a
 //                    bound on the segment's k-th largest (the k-th largest of the 256 threads'
